@@ -306,6 +306,10 @@ typedef struct {
 
 int mkx_modulation_input(const mkx_modin_args* args, void* stream);
 
+/* The same result through a workspace of N * H floats (16-byte aligned, overwritten; the launches of concurrent calls need
+ * one each): two launches, in which no workgroup reads more than 16 rows of a weight matrix. */
+int mkx_modulation_input_ws(const mkx_modin_args* args, float* ws, void* stream);
+
 /* Synchronisation micro-benchmarks (no handle). Reference: the barrier-only kernel _barrier_only
  * (src/tune_mk.py:28-33), timed at :66-68 to price the reference's grid barrier (results/opt/tune/v5.json:3-4).
  * MKX_PROBE_BARRIER: every workgroup of a one-per-CU grid passes n grid barriers (this library's barrier,

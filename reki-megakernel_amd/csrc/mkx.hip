@@ -888,6 +888,41 @@ int prep_rtw(int nrows, int ncol_groups, int ncu) {
 // Packed context bytes of a preparation of nrows rows (padded to a whole workgroup of the largest kind)
 long long prep_ctx_bytes(int nrows, int C) { return (long long)((nrows + 31) / 32 * 32 + PREP_ROW_PAD) * C * 2; }
 
+// Validation shared by mkx_modulation_input and mkx_modulation_input_ws.
+int modin_check(const mkx_modin_args* a, const char* who) {
+  const std::string w(who);
+  if (!a) return fail(MKX_EINVAL, w + ": args is NULL");
+  if (a->N < 1 || a->N > 4096 || a->B < 1 || a->B > (1 << 20))
+    return fail(MKX_EINVAL, w + ": need 1 <= N <= 4096 and B >= 1");
+  if (a->H != 256 && a->H != 512 && a->H != 768 && a->H != 1024)
+    return fail(MKX_EUNSUPPORTED, w + ": H must be 256, 512, 768 or 1024");
+  if (a->tdim < 32 || a->tdim > 32 * MODIN_MAX_TKB || (a->tdim & 31))
+    return fail(MKX_EUNSUPPORTED, w + ": tdim must be a multiple of 32 in [32, 512]");
+  if (a->sc_stride < a->H || (a->sc_stride & 3) || (a->out_stride_k & 3) || (a->out_stride_b & 3) ||
+      a->out_stride_k < a->H || (a->B > 1 && a->out_stride_b < (int64_t)a->N * a->out_stride_k))
+    return fail(MKX_EINVAL, w + ": strides must cover a row (and a sample) and be multiples of 4");
+  auto bad16 = [](const void* p) { return p == nullptr || ((uintptr_t)p & 15u) != 0; };
+  if (bad16(a->t1_w) || bad16(a->t1_b) || bad16(a->t2_w) || bad16(a->t2_b) || bad16(a->state_cond) || bad16(a->out))
+    return fail(MKX_EINVAL, w + ": a pointer is NULL or not 16-byte aligned");
+  return MKX_OK;
+}
+
+// The modulation projection of a.R rows: row groups of at most MODP_MAX_NRT row tiles, as even as they come (each
+// group streams the weights once more), one workgroup per CU and group, two per CU where one row tile leaves
+// the registers for it.
+template <int KT>
+void modproj_launch(const mkx_modproj_args& a, hipStream_t stream) {
+  const int nrt = (a.R + 15) / 16, ngr = (nrt + MODP_MAX_NRT - 1) / MODP_MAX_NRT, per = (nrt + ngr - 1) / ngr;
+  const dim3 grid((unsigned)std::min(a.N / 16, per == 1 ? 2 * MODP_GRID : MODP_GRID), (unsigned)((nrt + per - 1) / per)), block(64 * MODP_WAVES);
+  switch (per) {
+    case 1: hipLaunchKernelGGL((modproj_kernel<KT, 1>), grid, block, 0, stream, a); break;
+    case 2: hipLaunchKernelGGL((modproj_kernel<KT, 2>), grid, block, 0, stream, a); break;
+    case 3: hipLaunchKernelGGL((modproj_kernel<KT, 3>), grid, block, 0, stream, a); break;
+    case 4: hipLaunchKernelGGL((modproj_kernel<KT, 4>), grid, block, 0, stream, a); break;
+    default: hipLaunchKernelGGL((modproj_kernel<KT, 5>), grid, block, 0, stream, a); break;
+  }
+}
+
 // The two launches of a source preparation, the packed context staged at ctxp.
 int source_launch(const mkx_source* h, const mkx_source_args* a, bf16_t* ctxp, hipStream_t stream) {
   const mkx_source_dims& d = h->dims;
@@ -1019,32 +1054,40 @@ int mkx_modulations(const mkx_modproj_args* a, void* stream_) {
   if (bad16(a->c) || bad16(a->w) || bad16(a->bias) || bad16(a->out))
     return fail(MKX_EINVAL, "mkx_modulations: c, w, bias, out: NULL or not 16-byte aligned");
   hipStream_t stream = (hipStream_t)stream_;
-  const dim3 grid((unsigned)((a->N / 16 + 3) / 4)), block(MODP_BLOCK * MODP_KSPLIT);
   switch (a->K / 32) {
-    case 8: hipLaunchKernelGGL(modproj_kernel<8>, grid, block, modproj_lds_bytes<8>(), stream, *a); break;
-    case 16: hipLaunchKernelGGL(modproj_kernel<16>, grid, block, modproj_lds_bytes<16>(), stream, *a); break;
-    case 24: hipLaunchKernelGGL(modproj_kernel<24>, grid, block, modproj_lds_bytes<24>(), stream, *a); break;
-    default: hipLaunchKernelGGL(modproj_kernel<32>, grid, block, modproj_lds_bytes<32>(), stream, *a); break;
+    case 8: modproj_launch<8>(*a, stream); break;
+    case 16: modproj_launch<16>(*a, stream); break;
+    case 24: modproj_launch<24>(*a, stream); break;
+    default: modproj_launch<32>(*a, stream); break;
   }
   HIPCHK(hipGetLastError());
   return MKX_OK;
 }
 
 int mkx_modulation_input(const mkx_modin_args* a, void* stream_) {
-  if (!a) return fail(MKX_EINVAL, "mkx_modulation_input: args is NULL");
-  if (a->N < 1 || a->N > 4096 || a->B < 1 || a->B > (1 << 20))
-    return fail(MKX_EINVAL, "mkx_modulation_input: need 1 <= N <= 4096 and B >= 1");
-  if (a->H != 256 && a->H != 512 && a->H != 768 && a->H != 1024)
-    return fail(MKX_EUNSUPPORTED, "mkx_modulation_input: H must be 256, 512, 768 or 1024");
-  if (a->tdim < 32 || a->tdim > 32 * MODIN_MAX_TKB || (a->tdim & 31))
-    return fail(MKX_EUNSUPPORTED, "mkx_modulation_input: tdim must be a multiple of 32 in [32, 512]");
-  if (a->sc_stride < a->H || (a->sc_stride & 3) || (a->out_stride_k & 3) || (a->out_stride_b & 3) ||
-      a->out_stride_k < a->H || (a->B > 1 && a->out_stride_b < (int64_t)a->N * a->out_stride_k))
-    return fail(MKX_EINVAL, "mkx_modulation_input: strides must cover a row (and a sample) and be multiples of 4");
-  auto bad16 = [](const void* p) { return p == nullptr || ((uintptr_t)p & 15u) != 0; };
-  if (bad16(a->t1_w) || bad16(a->t1_b) || bad16(a->t2_w) || bad16(a->t2_b) || bad16(a->state_cond) || bad16(a->out))
-    return fail(MKX_EINVAL, "mkx_modulation_input: a pointer is NULL or not 16-byte aligned");
-  hipLaunchKernelGGL(modin_kernel, dim3((unsigned)(a->H / 64)), dim3(MODP_BLOCK), 0, (hipStream_t)stream_, *a);
+  const int rc = modin_check(a, "mkx_modulation_input");
+  if (rc != MKX_OK) return rc;
+  const dim3 grid((unsigned)(a->H / 64), (unsigned)((a->N + 15) / 16)), block(MODIN_BLOCK);
+  const size_t lds = (size_t)modin_lds_bytes(a->tdim, a->H);
+  hipStream_t stream = (hipStream_t)stream_;
+  switch (a->H / 256) {
+    case 1: hipLaunchKernelGGL(modin_kernel<1>, grid, block, lds, stream, *a); break;
+    case 2: hipLaunchKernelGGL(modin_kernel<2>, grid, block, lds, stream, *a); break;
+    case 3: hipLaunchKernelGGL(modin_kernel<3>, grid, block, lds, stream, *a); break;
+    default: hipLaunchKernelGGL(modin_kernel<4>, grid, block, lds, stream, *a); break;
+  }
+  HIPCHK(hipGetLastError());
+  return MKX_OK;
+}
+
+int mkx_modulation_input_ws(const mkx_modin_args* a, float* ws, void* stream_) {
+  const int rc = modin_check(a, "mkx_modulation_input_ws");
+  if (rc != MKX_OK) return rc;
+  if (!ws || ((uintptr_t)ws & 15u)) return fail(MKX_EINVAL, "mkx_modulation_input_ws: ws NULL or not 16-byte aligned");
+  const dim3 grid((unsigned)(a->H / 16), (unsigned)((a->N + 15) / 16)), block(64 * MODIN2_WAVES);
+  hipStream_t stream = (hipStream_t)stream_;
+  hipLaunchKernelGGL(modin_hidden_kernel, grid, block, 0, stream, *a, ws);
+  hipLaunchKernelGGL(modin_out_kernel, grid, block, 0, stream, *a, ws);
   HIPCHK(hipGetLastError());
   return MKX_OK;
 }

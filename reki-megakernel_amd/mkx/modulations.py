@@ -3,9 +3,9 @@
 AdaRMS scale, shift and gate of every layer and Euler step of a call — the rows the expert kernel reads
 (src/mk_expert.py:336-340).
 
-``StepModulations`` runs the whole of ``_step_modulations`` on this library's kernels: ``mkx_modulation_input``
-(the timestep embedding and the small MLP, c = silu(temb(t) W1^T + b1) W2^T + b2 + state_cond, one launch)
-and then the projection, two launches in all.
+``StepModulations`` runs the whole of ``_step_modulations`` on this library's kernels: ``mkx_modulation_input_ws``
+(the timestep embedding and the small MLP, c = silu(temb(t) W1^T + b1) W2^T + b2 + state_cond, two launches)
+and then the projection, three launches in all.
 
 ``ModulationProjection(weight, bias)`` keeps W as bf16 (repacked once into MFMA fragment order, so every
 weight load of the kernel is one contiguous 1 KB block per wave) and b as fp32 on the GPU; ``proj(c)`` runs
@@ -84,9 +84,10 @@ class StepModulations:
                          t1_b=self.t1_b.data_ptr(), t2_w=self.t2_w.data_ptr(), t2_b=self.t2_b.data_ptr(),
                          state_cond=sc.data_ptr(), sc_stride=self.H, out=out.data_ptr(),
                          out_stride_b=num_steps * self.H, out_stride_k=self.H)
-        check(lib().mkx_modulation_input(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
-              "mkx_modulation_input")
-        self._keep = sc  # the input outlives the asynchronous launch
+        ws = torch.empty(num_steps, self.H, dtype=torch.float32, device=self.device)  # the hidden layer
+        check(lib().mkx_modulation_input_ws(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()),
+                                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "mkx_modulation_input_ws")
+        self._keep = (sc, ws)  # the input and the workspace outlive the asynchronous launches
         return out
 
     def __call__(self, num_steps: int, state_cond: torch.Tensor):

@@ -161,3 +161,52 @@ def test_step_modulations_drive_the_expert_like_the_pytorch_ones():
     m, a = diff(x_k, x_t, cfg.action_dim)
     _report("expert on kernel step modulations vs PyTorch step modulations (A)", max=m, mean=a)
     assert m <= 1e-3 and a <= 2e-4
+
+
+def _rand(*shape, seed, std=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(*shape, generator=g) * std
+
+
+@pytest.mark.parametrize("fragment_order", [True, False])
+@pytest.mark.parametrize("R, K, N", [(1, 256, 16), (16, 768, 48), (17, 512, 4112), (33, 1024, 16 * 300), (48, 768, 16 * 257),
+                                     (49, 256, 16 * 513), (65, 768, 16 * 1030), (80, 1024, 16 * 700), (81, 512, 32),
+                                     (129, 768, 16 * 259), (161, 1024, 16)])
+def test_modulations_row_and_column_edges(R, K, N, fragment_order):
+    """Row tiles of every count a workgroup holds and more than one row group; fewer column tiles than workgroups,
+    and ranges that leave remainders of the weights' pipeline. Against 64 bits: silu(c) is held in two or
+    three bf16 parts (2^-18 relative at worst), a result is a sum of at most 3 K / 8 + 16 fp32 additions per wave and
+    over the waves, each rounded to 2^-24 of at most S = sum |silu(c) w| + |b|; the hardware exp and reciprocal add 2^-20."""
+    c, w, b = _rand(R, K + 12, seed=R)[:, :K], _rand(N, K, seed=K, std=0.02).bfloat16(), _rand(N, seed=N, std=0.02)
+    proj = ModulationProjection(w.cuda(), b.cuda(), fragment_order=fragment_order)
+    out = proj(c.cuda()).cpu().double()
+    a = torch.nn.functional.silu(c.double())
+    ref = a @ w.double().T + b.double()
+    S = a.abs() @ w.double().abs().T + b.double().abs()
+    bound = (2.0 ** -18 + 2.0 ** -20 + (3 * K / 8 + 16) * 2.0 ** -24) * S
+    assert bool(((out - ref).abs() <= bound).all()), float(((out - ref).abs() / S).max())
+
+
+@pytest.mark.parametrize("N, B, H, tdim", [(1, 1, 256, 32), (10, 1, 768, 256), (15, 5, 512, 64), (16, 2, 768, 160), (17, 3, 1024, 512),
+                                           (33, 6, 1024, 96)])
+def test_modulation_input_step_and_width_edges(N, B, H, tdim):
+    """Steps below, at and past a row tile of 16, every width, odd k-block counts of the embedding and more samples than
+    waves share a column tile. Against 64 bits, with the error carried through: embedding rounded to fp32 (2^-24), sums of
+    n fp32 additions (n 2^-24 of the sum of magnitudes), silu (slope at most 1.1; hardware exp 2^-20)."""
+    bf = torch.bfloat16
+    t1w, t2w = _rand(H, tdim, seed=1, std=0.05).to(bf), _rand(H, H, seed=2, std=0.05).to(bf)
+    t1b, t2b, sc = _rand(H, seed=3, std=0.1), _rand(H, seed=4, std=0.1), _rand(B, H, seed=5)
+    step = StepModulations(t1w.cuda(), t1b.cuda(), t2w.cuda(), t2b.cuda(), _rand(16, H, seed=6).to(bf).cuda(), _rand(16, seed=7).cuda())
+    out = step.input(N, sc.cuda()).cpu().double()
+    d = torch.float64
+    half = tdim // 2
+    arg = 1000.0 * (1.0 - torch.arange(N, dtype=d) / N)[:, None] * 10000.0 ** (-torch.arange(half, dtype=d) / half)
+    temb = torch.cat([torch.cos(arg), torch.sin(arg)], -1)
+    pre = temb @ t1w.to(d).T + t1b.to(d)
+    h1 = torch.nn.functional.silu(pre)
+    ref = (h1 @ t2w.to(d).T + t2b.to(d))[None] + sc.to(d)[:, None]
+    e_pre = (3 * tdim + 8) * 2.0 ** -24 * (temb.abs() @ t1w.to(d).abs().T + t1b.to(d).abs())
+    e_h1 = 1.1 * e_pre + 2.0 ** -20 * h1.abs()
+    bound = e_h1 @ t2w.to(d).abs().T + (3 * H / 4 + 16) * 2.0 ** -24 * (h1.abs() @ t2w.to(d).abs().T + t2b.to(d).abs())
+    bound = bound[None] + 2.0 ** -22 * (1.0 + sc.to(d).abs()[:, None])
+    assert bool(((out - ref).abs() <= bound).all()), float((out - ref).abs().max())

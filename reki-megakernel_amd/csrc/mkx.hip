@@ -871,17 +871,18 @@ int source_args_check(const mkx_source* h, const mkx_source_args* a, const char*
   return MKX_OK;
 }
 
-// Row tiles per wave of prepare_source_kernel for nrows source rows on ncu compute units: the one whose
-// busiest CU has the least work, counting a workgroup's fixed cost (its first k-blocks in flight, the
-// epilogue) as one row tile.
-int prep_rtw(int nrows, int ncol_groups, int ncu) {
+// Row tiles per workgroup of prepare_source_kernel for nrows source rows on ncu compute units: the count whose
+// busiest CU has the least work, counting a workgroup's fixed cost (its first fragments in flight, the sum over the
+// waves and the epilogue) as PREP_FIXED row tiles.
+constexpr int PREP_FIXED = 4;
+int prep_nrt(int nrows, int ncol_groups, int ncu) {
   const int nrt = (nrows + 15) / 16;
   int best = 2;
   long long best_cost = -1;
-  for (int rtw = 2; rtw <= 5; ++rtw) {
-    const long long nwg = (long long)((nrt + 2 * rtw - 1) / (2 * rtw)) * ncol_groups;
-    const long long cost = (nwg + ncu - 1) / ncu * (rtw + 1);
-    if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = rtw; }
+  for (int n = 2; n <= 5; ++n) {
+    const long long nwg = (long long)((nrt + n - 1) / n) * ncol_groups;
+    const long long cost = (nwg + ncu - 1) / ncu * (n + PREP_FIXED);
+    if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = n; }
   }
   return best;
 }
@@ -928,32 +929,27 @@ int source_launch(const mkx_source* h, const mkx_source_args* a, bf16_t* ctxp, h
   const mkx_source_dims& d = h->dims;
   const int nrows = a->B * a->SP;
   const int np = (d.NH + 1) / 2, ncg = d.L * 2 * np;
-  const int rtw = prep_rtw(nrows, ncg, h->ncu), wg_rows = 32 * rtw;
+  const int nrt = prep_nrt(nrows, ncg, h->ncu), wg_rows = 16 * nrt;
   const int ngroups = (nrows + wg_rows - 1) / wg_rows;
   // packed pieces: rows padded with zeros to whole workgroups
   const long long n_x = (long long)ngroups * wg_rows * d.C / 8;
-  // packed in groups of a workgroup's 2 rtw row tiles, so that one k-block of a workgroup's rows is contiguous
-  hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)((n_x + 255) / 256)), dim3(256), 0, stream, (const bf16_t*)a->ctx,
-                     ctxp, nrows, d.C, 2 * rtw, n_x);
+  // packed in groups of a workgroup's row tiles, so that one k-block of a workgroup's rows is contiguous
+  hipLaunchKernelGGL(pack_ctx_kernel, dim3((unsigned)((n_x + 255) / 256)), dim3(256), 0, stream, (const bf16_t*)a->ctx,
+                     ctxp, a->ca_len, a->B, a->SP, d.C, nrt, n_x);
   SourceParams p{};
   p.L = d.L; p.NH = d.NH; p.C = d.C; p.B = a->B; p.SP = a->SP;
+  p.sbw = (int)std::max(1LL, PREP_L2_CTX / ((long long)wg_rows * d.C * 2));
   p.ctxp = ctxp; p.wkp = h->wkp; p.wvp = h->wvp; p.k_norm = h->kn;
   p.ca_len = a->ca_len; p.cos = a->cos; p.sin = a->sin;
   for (int l = 0; l < d.L; ++l) { p.kca[l] = a->kca[l]; p.vca[l] = a->vca[l]; }
   p.src_sb = a->src_stride_b;
   p.eps = d.eps;
   const dim3 grid((unsigned)ngroups, (unsigned)ncg);
-  // the production context width (2048) runs the fully unrolled k-loop
-  const bool c2048 = d.C == 2048;
-  switch (rtw) {
-    case 2: if (c2048) hipLaunchKernelGGL((prepare_source_kernel<2, 64>), grid, dim3(PREP_BLOCK), 0, stream, p);
-            else hipLaunchKernelGGL((prepare_source_kernel<2, 0>), grid, dim3(PREP_BLOCK), 0, stream, p); break;
-    case 3: if (c2048) hipLaunchKernelGGL((prepare_source_kernel<3, 64>), grid, dim3(PREP_BLOCK), 0, stream, p);
-            else hipLaunchKernelGGL((prepare_source_kernel<3, 0>), grid, dim3(PREP_BLOCK), 0, stream, p); break;
-    case 4: if (c2048) hipLaunchKernelGGL((prepare_source_kernel<4, 64>), grid, dim3(PREP_BLOCK), 0, stream, p);
-            else hipLaunchKernelGGL((prepare_source_kernel<4, 0>), grid, dim3(PREP_BLOCK), 0, stream, p); break;
-    default: if (c2048) hipLaunchKernelGGL((prepare_source_kernel<5, 64>), grid, dim3(PREP_BLOCK), 0, stream, p);
-             else hipLaunchKernelGGL((prepare_source_kernel<5, 0>), grid, dim3(PREP_BLOCK), 0, stream, p); break;
+  switch (nrt) {
+    case 2: hipLaunchKernelGGL(prepare_source_kernel<2>, grid, dim3(PREP_BLOCK), 0, stream, p); break;
+    case 3: hipLaunchKernelGGL(prepare_source_kernel<3>, grid, dim3(PREP_BLOCK), 0, stream, p); break;
+    case 4: hipLaunchKernelGGL(prepare_source_kernel<4>, grid, dim3(PREP_BLOCK), 0, stream, p); break;
+    default: hipLaunchKernelGGL(prepare_source_kernel<5>, grid, dim3(PREP_BLOCK), 0, stream, p); break;
   }
   HIPCHK(hipGetLastError());
   return MKX_OK;

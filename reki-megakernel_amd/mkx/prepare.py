@@ -96,18 +96,18 @@ class SourcePrepare:
         cal = torch.as_tensor(ca_len, dtype=torch.int32).reshape(-1).to(dev).contiguous()
         if cal.numel() != B:
             raise ValueError("ca_len needs one entry per sample")
-        ks = [torch.empty(B, SP, self.NH, 64, dtype=torch.bfloat16, device=dev) for _ in range(self.L)]
-        vs = [torch.empty_like(ks[0]) for _ in range(self.L)]
+        # every layer's K and V in one allocation (2 L of them took longer on the host than the launches run)
+        kv = torch.empty(2, self.L, *((B,) if batched else ()), SP, self.NH, 64, dtype=torch.bfloat16, device=dev)
+        base, step = kv.data_ptr(), B * SP * self.NH * 64 * 2
         a = MkxSourceArgs(B=B, SP=SP)
         a.ctx, a.ca_len = x.data_ptr(), cal.data_ptr()
         a.cos, a.sin = cos.data_ptr(), sin.data_ptr()
         for l in range(self.L):
-            a.kca[l], a.vca[l] = ks[l].data_ptr(), vs[l].data_ptr()
+            a.kca[l], a.vca[l] = base + l * step, base + (self.L + l) * step
         a.src_stride_b = SP * self.NH * 64
         fn = lib().mkx_source_run_noalloc if static_scratch else lib().mkx_source_run
         check(fn(self._h, ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
               "mkx_source_run_noalloc" if static_scratch else "mkx_source_run")
         self._keep = (x, cal, cos, sin)  # inputs outlive the asynchronous launch
-        if batched:
-            return list(zip(ks, vs))
-        return [(k[0], v[0]) for k, v in zip(ks, vs)]
+        ks, vs = kv.unbind(0)
+        return list(zip(ks.unbind(0), vs.unbind(0)))

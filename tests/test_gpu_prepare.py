@@ -75,6 +75,34 @@ def test_prepare_wide_expert():
     _check_prepare("prepare D shape (NH16, 4 layers)", cfg)
 
 
+@pytest.mark.parametrize("B, SP, C, lens", [
+    (1, 5, 32, [5]),                         # one k-block: three of the four waves have none
+    (3, 37, 160, [37, 0, 20]),               # an empty sample between others; waves with one and with two k-blocks
+    (2, 64, 288, [64, 48]),                  # whole row tiles; nine k-blocks
+    (5, 31, 96, [1, 31, 16, 17, 30]),        # samples that end inside, at and past a row tile
+    (66, 3, 64, [b % 4 for b in range(66)]),  # more samples than are numbered densely
+    (64, 3, 64, [(3 * b) % 4 for b in range(64)]),
+    (1, 600, 96, [333]),                     # fewer valid rows than row groups launched
+    (4, 300, 4096, [300, 300, 299, 41]),     # more than one block of row groups
+    (2, 1024, 2048, [1000, 3]),
+])
+def test_prepare_numbered_rows(B, SP, C, lens):
+    """Valid rows are numbered densely over up to 64 samples and the rows past each sample's length zeroed by the row
+    groups' workgroups; k-blocks are dealt over the waves. The tolerance is the module's (one bf16 rounding)."""
+    _check_prepare(f"prepare B {B}, SP {SP}, C {C}", replace(TINY, B=B, S=SP, SP=SP, ctx_dim=C), ca_len=lens)
+
+
+@pytest.mark.parametrize("B", [2, 70])
+def test_prepare_clamps_lengths(B):
+    """Lengths outside [0, SP] give the same bits as the clamped ones, densely numbered (2 samples) or not (70)."""
+    cfg = replace(TINY, B=B, S=33, SP=33)
+    prep = SourcePrepare(SY.SyntheticReki(cfg, SY.make_weights(cfg, 0), device="cuda"))
+    ctx = SY.make_inputs(cfg)["ctx"].cuda()
+    wild = [(-2, 40)[b % 2] for b in range(B)]
+    for (k0, v0), (k1, v1) in zip(prep(ctx, wild), prep(ctx, [min(max(n, 0), 33) for n in wild])):
+        assert torch.equal(k0, k1) and torch.equal(v0, v1)
+
+
 def test_expert_on_kernel_prepared_caches():
     """Euler steps 2..N on caches from the kernel: within the tight bound of the fp32 oracle run on the
     same caches, and close to the run on the PyTorch-prepared caches."""

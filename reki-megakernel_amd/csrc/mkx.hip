@@ -38,6 +38,22 @@ int fail(int code, const std::string& msg) {
 constexpr unsigned SPIN_LIMIT = 1u << 20;  // default spin bound of a wait (polls), about 0.5 s
 constexpr int MAX_ROWS_PADDED = 512;
 
+// The multipliers of mdiv() give the quotient for every row, tile and task index of a launch: a quotient only changes at
+// the multiples of d, so x = k d - 1 and x = k d are checked.
+constexpr bool mdiv_exact(int d, int x_max) {
+  const uint32_t m = mdiv_m(d);
+  for (int x = d; x <= x_max + d; x += d)
+    if (mdiv<true>(x - 1, m, d) != x / d - 1 || mdiv<true>(x, m, d) != x / d) return false;
+  return mdiv<true>(0, m, d) == 0;
+}
+constexpr bool mdiv_exact_upto(int d_max, int x_max, bool times_d) {
+  for (int d = 1; d <= d_max; ++d)
+    if (!mdiv_exact(d, times_d ? x_max * d : x_max)) return false;
+  return true;
+}
+static_assert(mdiv_exact_upto(256, FLAG_MAX, false), "tasks by tiles; rows by a sample's rows or row tiles; row tiles by row groups");
+static_assert(mdiv_exact_upto(24, MAX_ROWS_PADDED, true), "(row, action dim) items by action dims");
+
 // W [L][N][K] row-major bf16 -> fp16 chunks (l, t, kb): dst[l*dls + (t'*tstride + toff + kb)*512 + lane*8 + j]
 // = W[l][t*16 + lane%16][kb*32 + 8(lane/16) + j] (the MFMA 16x16x32 operand layout). t' = t, or with
 // `pairs` the 16-column tiles of each 64-column head reordered 0, 2, 1, 3 (a task's d and d + 32 tiles
@@ -746,6 +762,9 @@ int mkx_run(mkx_handle* h, const mkx_step_args* a, void* stream_) {
   p.nt_o = lay.nt_o; p.nt_cao = lay.nt_cao; p.nt_down = lay.nt_down;
   p.lds_red = lay.lds_red; p.lds_mods = lay.lds_mods;
   p.tpr = lay.tpr; p.nred = lay.nred; p.nrg = lay.nrg;
+  p.m_mqp = mdiv_m(Mqp); p.m_nqt = mdiv_m(Mqp / 16); p.m_RT = mdiv_m(NRP / 16); p.m_T = mdiv_m(a->T_act);
+  p.m_adim = mdiv_m(a->action_dim); p.m_rgs_qkv = mdiv_m(lay.rgs_qkv); p.m_rgs_o = mdiv_m(lay.rgs_o);
+  p.m_rgs_cao = mdiv_m(lay.rgs_cao);
   bool pairs;
   {
     // attention tasks of two query tiles (row-wise form): where the one-tile tasks outnumber the workgroups and

@@ -106,6 +106,8 @@ struct Params {
   // row-wise form: cross-attention tasks of two query tiles (ca_stage_pairs; the self-attention ones are the
   // Shape::PAIRS instantiations')
   int ca_grp;
+  // multipliers of mdiv() for the launch's divisors: Mqp, Mqp / 16, NRP / 16, T, action_dim and the row groups
+  uint32_t m_mqp, m_nqt, m_RT, m_T, m_adim, m_rgs_qkv, m_rgs_o, m_rgs_cao;
 };
 
 // placement kinds (Params::pl)
@@ -116,6 +118,12 @@ enum { PL_QKV = 0, PL_SA, PL_O, PL_CA, PL_CAO, PL_GU, PL_DOWN, PL_RED, PL_TIN, P
 typedef const __attribute__((address_space(4))) Params CP;
 
 __host__ __device__ constexpr int ceil_to(int a, int m) { return (a + m - 1) / m * m; }
+
+// x / d, x >= 0: by the multiplier m = mdiv_m(d) (ON; exact while x d < 2^20 and x m < 2^32, far above a launch's
+// rows, tiles and tasks), or by dividing
+__host__ __device__ constexpr uint32_t mdiv_m(int d) { return (1u << 20) / (uint32_t)(d > 0 ? d : 1) + 1; }
+template <bool ON>
+__host__ __device__ constexpr int mdiv(int x, uint32_t m, int d) { return ON ? (int)(((uint32_t)x * m) >> 20) : x / d; }
 
 template <int H_, int I_, bool W8_ = false, bool RW_ = false, bool YS_ = false, bool PR_ = false, bool LS_ = false>
 struct Shape {
@@ -130,6 +138,13 @@ struct Shape {
   // measured slower with them, also for launches that never run the pairs (workload D 7.65 -> 7.86 ms and
   // D-b4 12.79 -> 13.00 ms with the pairs; 7.65 -> 7.69 and 12.77 -> 12.86 ms with the late K/V DMA).
   static constexpr bool RW_ATTN = RW_ && !W8_;
+  // MDIV: task, row and tile indices are split by multipliers of the launch (mdiv) instead of divisions, some 30 dependent
+  // instructions each. In the row-wise form nearly every workgroup runs every GEMM stage, so this work lies between one
+  // task's end and the next one's poll: with the shift fragments' loads ahead of the poll D 6.74 -> 6.48, D-b4 11.79 ->
+  // 11.46, B's ten steps 6.30 -> 6.12 ms (the loads alone: 6.66, 11.86 and 6.27). In the form with passes, whose
+  // transitions are off the critical path, it measured 2.70 -> 2.72 ms and more; the attention stages' task order by
+  // multipliers made B 2 % slower.
+  static constexpr bool MDIV = RW_;
   // CA_LATE: cross-attention DMAs its source K/V after its ready-epoch poll and query rows: the fp16 row-wise
   // instantiations and the two-tile ones (not the other fp8 row-wise ones, whose launches, workload D, measured
   // 7.59 -> 7.74 ms with it)
@@ -291,7 +306,7 @@ struct Ctx {
     return p.mods + (long long)b * p.mods_sb + (long long)(p.mod_row0 + s) * p.mods_ss;
   }
   __device__ int sample_of(int grow) const {
-    int b = grow / p.Mqp;
+    int b = mdiv<S::MDIV>(grow, p.m_mqp, p.Mqp);
     return b < p.B ? b : p.B - 1;
   }
 };
@@ -452,8 +467,9 @@ __device__ __forceinline__ int task_first(Ctx<S>& c, int k) {
   return t < 0 ? t + c.G : t;
 }
 
-// row group (of rgs over RT row tiles, group g covering [g RT / rgs, (g + 1) RT / rgs)) holding row tile rt
-__device__ __forceinline__ int row_group_of(int rt, int RT, int rgs) { return ((rt + 1) * rgs - 1) / RT; }
+// row group (of rgs over the RT row tiles, group g covering [g RT / rgs, (g + 1) RT / rgs)) holding row tile rt
+template <class S>
+__device__ __forceinline__ int row_group_of(Ctx<S>& c, int rt, int rgs) { return mdiv<S::MDIV>((rt + 1) * rgs - 1, c.p.m_RT, c.RT); }
 
 // ------------------------------------------------------------------------------------------------
 // Stage descriptor: what one stage computes, where its operands live, and what to prefetch for it.
@@ -470,6 +486,7 @@ struct Desc {
   const float* ssin;                   // AdaRMS stages: the operand's sums of squares [RT][HT / 2][16][2]
   int ntask, tiles, kind, nt;          // nt: 16-column tiles per task (QKV, gate/up: a pair; wide tasks: NTW)
   int rgs;                             // row groups: task t = tile t % tiles over row-tile group t / tiles
+  uint32_t m_tiles, m_rgs;             // mdiv multipliers of tiles and rgs
   int pk;                              // placement kind (Params::pl)
   const char* shs;                     // AdaRMS stages: the fp16 shift fragments of this step and layer
   // staged modulation slices (H floats each, per sample): AdaRMS stages: shift; residual stages: gate, then
@@ -504,6 +521,7 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
   d.sc = nullptr; d.sc2 = nullptr;
   d.yout = nullptr; d.ssout = nullptr; d.ssin = nullptr; d.shs = nullptr;
   d.ntask = 0; d.tiles = 1; d.kind = K_QKV; d.nt = 1; d.mod_off = 0; d.mod_off2 = 0; d.rgs = 1; d.pk = PL_TIN;
+  d.m_tiles = d.m_rgs = mdiv_m(1);
   if (q.g == 0) { d.st = ST_TAIL; d.s = 0; d.l = 0; return d; }
   d.s = q.s;
   if (q.l == p.L) {
@@ -525,14 +543,15 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
       if (S::W8) d.sc = p.sc_qkv + (long long)l * 3 * S::H;
       d.out = (float*)(fr + S::qs_off(NRP)); d.yout = (float*)(fr + S::ks_off(NRP)); d.part = (float*)(fr + S::vtb_off(NRP));
       d.ssout = (float*)(fr + S::ssqk_off(NRP)); d.tiles = 6 * S::NH; d.nt = 2; d.shs = shs;
-      d.rgs = p.rgs_qkv; d.pk = PL_QKV;
+      d.rgs = p.rgs_qkv; d.pk = PL_QKV; d.m_tiles = mdiv_m(6 * S::NH); d.m_rgs = p.m_rgs_qkv;
       break;
     case ST_O:
       d.w = p.wo + l * p.s_o; d.a = (const float*)(fr + S::ysa_off(NRP)); d.out = (float*)(fr + S::h2_off(NRP));
       if (S::W8) d.sc = p.sc_o + (long long)l * S::H;
       d.yout = (float*)(fr + S::y2_off(NRP)); d.ssout = (float*)(fr + S::ss2_off(NRP));
       d.res = c.h_in(d.s, l); d.kind = K_RES; d.mod_off = m_sa + 2 * S::H; d.mod_off2 = m_ca;
-      d.nt = p.nt_o; d.tiles = S::HT / d.nt; d.wstride = (long long)d.nt * S::NKB * S::CH; d.rgs = p.rgs_o; d.pk = PL_O;
+      d.nt = p.nt_o; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.wstride = (long long)d.nt * S::NKB * S::CH;
+      d.m_tiles = mdiv_m(S::HT); d.rgs = p.rgs_o; d.m_rgs = p.m_rgs_o; d.pk = PL_O;
       break;
     case ST_CAO:
       d.w = p.woca + l * p.s_o; d.a = (const float*)(fr + S::yca_off(NRP)); d.out = (float*)(fr + S::h3_off(NRP));
@@ -540,20 +559,21 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
       d.yout = (float*)(fr + S::y3_off(NRP)); d.ssout = (float*)(fr + S::ss3_off(NRP));
       d.res = (const float*)(fr + S::h2_off(NRP)); d.kind = K_RES;
       d.mod_off = m_ca + 2 * S::H; d.mod_off2 = m_mlp;
-      d.nt = p.nt_cao; d.tiles = S::HT / d.nt; d.wstride = (long long)d.nt * S::NKB * S::CH; d.rgs = p.rgs_cao; d.pk = PL_CAO;
+      d.nt = p.nt_cao; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.wstride = (long long)d.nt * S::NKB * S::CH;
+      d.m_tiles = mdiv_m(S::HT); d.rgs = p.rgs_cao; d.m_rgs = p.m_rgs_cao; d.pk = PL_CAO;
       break;
     case ST_GU:
       d.w = p.wgu + l * p.s_gu; d.wstride = 2LL * S::NKB * S::CH; d.a = (const float*)(fr + S::y3_off(NRP));
       if (S::W8) { d.sc = p.sc_g + (long long)l * S::I; d.sc2 = p.sc_u + (long long)l * S::I; }
       d.ssin = (const float*)(fr + S::ss3_off(NRP)); d.out = (float*)(fr + S::g_off(NRP));
-      d.tiles = S::IT; d.kind = K_GU; d.nt = 2; d.shs = shs + 2 * p.B * S::H * 4; d.pk = PL_GU;
+      d.tiles = S::IT; d.m_tiles = mdiv_m(S::IT); d.kind = K_GU; d.nt = 2; d.shs = shs + 2 * p.B * S::H * 4; d.pk = PL_GU;
       break;
     case ST_DOWN:
       d.w = p.wd + l * p.s_d; d.a = (const float*)(fr + S::g_off(NRP)); d.out = (float*)(fr + S::hl_off(NRP));
       if (S::W8) d.sc = p.sc_d + (long long)l * S::H;
       d.yout = (float*)(fr + S::yl_off(NRP)); d.ssout = (float*)(fr + S::ssl_off(NRP));
       d.res = (const float*)(fr + S::h3_off(NRP)); d.part = (float*)(fr + S::part_off(NRP));
-      d.nt = p.nt_down; d.tiles = S::HT / d.nt; d.rgs = S::SK; d.kind = K_SPLIT; d.pk = PL_DOWN;
+      d.nt = p.nt_down; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.m_tiles = mdiv_m(S::HT); d.rgs = S::SK; d.kind = K_SPLIT; d.pk = PL_DOWN;
       d.mod_off = m_mlp + 2 * S::H; d.mod_off2 = m_next;
       break;
     case ST_SA:
@@ -573,7 +593,7 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
 // down projection's splits are packed [tile][split][k-block], so its tiles are nt runs)
 template <class S>
 __device__ __forceinline__ void dma_task_w(Ctx<S>& c, const Desc& d, int t, char* dst) {
-  const int tile = t % d.tiles, split = t / d.tiles;
+  const int split = mdiv<S::MDIV>(t, d.m_tiles, d.tiles), tile = S::MDIV ? t - split * d.tiles : t % d.tiles;
   if (d.kind == K_SPLIT) {
     for (int j = 0; j < d.nt; ++j)
       dma_w(c, dst + j * S::NKB * S::CH, d.w + ((long long)(tile * d.nt + j) * S::SK + split) * S::NKB * S::CH,
@@ -890,10 +910,11 @@ __device__ __forceinline__ void gemm_wait(Ctx<S>& c, const Desc& d, BarCtx& bc, 
   } else if (d.st == ST_O || d.st == ST_CAO) {
     flag_wait(bc, d.st == ST_O ? F_SA : F_CA, (rt_hi - rt_lo) * S::NH, [&](int i) {
       const int rt = rt_lo + i / S::NH, hd = i % S::NH;
-      return ((rt / NQT) * S::NH + hd) * NQT + rt % NQT;
+      const int sm = mdiv<S::MDIV>(rt, c.p.m_nqt, NQT);
+      return (sm * S::NH + hd) * NQT + (S::MDIV ? rt - sm * NQT : rt % NQT);
     }, (unsigned long long)g);
   } else if (d.st == ST_GU) {
-    flag_wait(bc, F_CAO, (S::HT / c.p.nt_cao) * c.p.rgs_cao, [](int i) { return i; }, (unsigned long long)g);
+    flag_wait(bc, F_CAO, (S::RW ? S::HT : S::HT / c.p.nt_cao) * c.p.rgs_cao, [](int i) { return i; }, (unsigned long long)g);
   } else {
     flag_wait<1>(bc, F_GU, S::HT, [&](int i) { return split * S::HT + i; }, (unsigned long long)g);
   }
@@ -914,15 +935,15 @@ __device__ __forceinline__ void down_reduce(Ctx<S>& c, const Desc& d, BarCtx& bc
   if constexpr (S::RW) {
     const int rgr = r / S::HT;
     t0 = (r % S::HT) * tpr;
-    rlo = rgr * RT / c.p.nrg;
-    nrt = (rgr + 1) * RT / c.p.nrg - rlo;
+    rlo = mdiv<S::MDIV>(rgr * RT, c.p.m_rgs_qkv, c.p.nrg);  // (nrg: the QKV stage's row groups)
+    nrt = mdiv<S::MDIV>((rgr + 1) * RT, c.p.m_rgs_qkv, c.p.nrg) - rlo;
   } else {
     t0 = r * tpr;
     rlo = 0;
     nrt = RT;
   }
   // the tile groups (split tasks per split) holding tiles t0 .. t0 + tpr - 1
-  const int g0 = t0 / d.nt, ng = (t0 + tpr - 1) / d.nt - g0 + 1;
+  const int nt = S::RW ? 1 : d.nt, g0 = t0 / nt, ng = (t0 + tpr - 1) / nt - g0 + 1;
   flag_wait<1>(bc, F_DPART, S::SK * ng, [&](int i) { return (i % S::SK) * d.tiles + g0 + i / S::SK; }, (unsigned long long)g);
   wait_vm0();  // the staged gate and next AdaRMS scale (the prefetch's DMA) have landed
   __syncthreads();
@@ -936,7 +957,7 @@ __device__ __forceinline__ void down_reduce(Ctx<S>& c, const Desc& d, BarCtx& bc
 #pragma unroll
     for (int k = 0; k < RR; ++k) {
       const int blk = min(b0 + NWAVES * k, nblk - 1);
-      const int tile = t0 + blk / nrt, rtg = rlo + blk % nrt, L = c.lane;
+      const int tile = t0 + (S::RW ? 0 : blk / nrt), rtg = rlo + (S::RW ? blk : blk % nrt), L = c.lane;  // (RW: one tile)
 #pragma unroll
       for (int j = 0; j < S::SK; ++j) xp[k][j] = ld16((const char*)d.part + ((((j * S::HT + tile) * RT + rtg) * 64 + L) * 16));
       res[k] = as_f4(ld16((const char*)d.res + fpiece(rtg * 16 + (L & 15), tile * 16 + 4 * (L >> 4), RT)));
@@ -945,7 +966,7 @@ __device__ __forceinline__ void down_reduce(Ctx<S>& c, const Desc& d, BarCtx& bc
     for (int k = 0; k < RR; ++k) {
       const int blk = b0 + NWAVES * k;
       if (blk >= nblk) break;
-      const int tile = t0 + blk / nrt, rtg = rlo + blk % nrt, L = c.lane;
+      const int tile = t0 + (S::RW ? 0 : blk / nrt), rtg = rlo + (S::RW ? blk : blk % nrt), L = c.lane;  // (RW: one tile)
       const int row = rtg * 16 + (L & 15), col = tile * 16 + 4 * (L >> 4);
       f32x4 v = as_f4(xp[k][0]);
 #pragma unroll
@@ -1344,7 +1365,7 @@ __device__ __forceinline__ void gemm_stage_rows(Ctx<S>& c, const Desc& d, BarCtx
   const bool ada = d.kind == K_QKV || d.kind == K_GU;
   const int t0 = task_first(c, d.pk);
   for (int t = t0; t < d.ntask; t += c.G) {
-    const int tile = t % d.tiles, split = t / d.tiles;
+    const int split = mdiv<S::MDIV>(t, d.m_tiles, d.tiles), tile = t - split * d.tiles;
     const int qkind = d.kind == K_QKV ? tile / (2 * S::NH) : 0, qhd = (tile >> 1) % S::NH, qj = tile & 1;
     if (t != t0) {
       wait_vm0();
@@ -1353,18 +1374,10 @@ __device__ __forceinline__ void gemm_stage_rows(Ctx<S>& c, const Desc& d, BarCtx
       if (d.kind == K_RES) dma_mods_tile(c, d, tile);
     }
     const int kb0 = d.kind == K_SPLIT ? split * NKB : 0;
-    const int rt_lo = d.kind == K_SPLIT ? 0 : split * RT / d.rgs;
-    const int rt_hi = d.kind == K_SPLIT ? RT : (split + 1) * RT / d.rgs;
-    MKX_TR(c, 14);
-    gemm_wait(c, d, bc, g, split, rt_lo, rt_hi);
-    MKX_TR(c, 0);
-    // the task's weight tiles (and a gated-residual task's modulation slices: the prefetch's DMA) have landed
-    wait_vm0();
-    __syncthreads();
-    MKX_TR(c, 1);
+    const int rt_lo = d.kind == K_SPLIT ? 0 : mdiv<S::MDIV>(split * RT, d.m_rgs, d.rgs);
+    const int rt_hi = d.kind == K_SPLIT ? RT : mdiv<S::MDIV>((split + 1) * RT, d.m_rgs, d.rgs);
     // AdaRMS tasks: the fp16 shift fragments of this wave's k-blocks (lane l: sample l % 16, zeros for the
-    // samples >= B), loaded from the launch's copy after the poll rather than staged in LDS ahead of it (the
-    // poll returns only after every load issued before it), and before the operand loads, so they land first
+    // samples >= B), loaded ahead of the poll, so that they land while the task waits
     f16x8 shv[KPW];
     if (ada) {
       const bool has = (L & 15) < p.B;
@@ -1375,6 +1388,13 @@ __device__ __forceinline__ void gemm_stage_rows(Ctx<S>& c, const Desc& d, BarCtx
         shv[i] = has ? v : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
       }
     }
+    MKX_TR(c, 14);
+    gemm_wait(c, d, bc, g, split, rt_lo, rt_hi);
+    MKX_TR(c, 0);
+    // the task's weight tiles (and a gated-residual task's modulation slices: the prefetch's DMA) have landed
+    wait_vm0();
+    __syncthreads();
+    MKX_TR(c, 1);
     // the operand loads of this wave's first group go out before the shift tile
     const int ng = (rt_hi - rt_lo + NR - 1) / NR;
     const __amdgpu_buffer_rsrc_t ra = rsrc(d.a);
@@ -2286,8 +2306,8 @@ __device__ __forceinline__ void ca_stage(Ctx<S>& c, const Desc& d, const int* s_
     MKX_TR(c, 14);
     // every out-projection task of the row group holding the query rows
     {
-      const int rg = row_group_of(rq, RT, rgo);
-      const int to = S::HT / p.nt_o;  // out-projection tasks per row group
+      const int rg = row_group_of(c, rq, rgo);
+      const int to = S::RW ? S::HT : S::HT / p.nt_o;  // out-projection tasks per row group
       flag_wait<1>(bc, F_O, to, [&](int i) { return rg * to + i; }, (unsigned long long)g);
     }
     MKX_TR(c, 0);
@@ -3133,8 +3153,8 @@ __device__ __forceinline__ void ca_stage_pairs(Ctx<S>& c, const Desc& d, const i
   // every out-projection task of the row groups holding the two tiles' rows
   const int rq0 = b * Mqp / 16 + qa, rq1 = rq0 + nq - 1;
   {
-    const int to = S::HT / p.nt_o;
-    const int rg0 = row_group_of(rq0, RT, p.rgs_o), rg1 = row_group_of(rq1, RT, p.rgs_o);
+    const int to = S::RW ? S::HT : S::HT / p.nt_o;
+    const int rg0 = row_group_of(c, rq0, p.rgs_o), rg1 = row_group_of(c, rq1, p.rgs_o);
     flag_wait<1>(bc, F_O, to, [&](int i) { return rg0 * to + i; }, (unsigned long long)g);
     if (rg1 != rg0) flag_wait<1>(bc, F_O, to, [&](int i) { return rg1 * to + i; }, (unsigned long long)g);
   }
@@ -3404,7 +3424,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
     if (!d.first && S::RW && inproj) {
       const float* xn = c.xstep(d.s + 1);
       for (int it = c.tid; it < nrows * adim; it += NTHREADS) {
-        const int ri = it / adim, a = it - ri * adim;
+        const int ri = mdiv<S::MDIV>(it, p.m_adim, adim), a = it - ri * adim;
         xp[it] = xn[(long long)ri * p.A + a];
       }
     } else if (!d.first) {
@@ -3433,7 +3453,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
 #pragma unroll
         for (int k = 0; k < R; ++k) {
           const int ri = min(r0 + NWAVES * k, r_hi - 1);
-          const int b = ri / p.T, grow = b * p.Mqp + (ri - b * p.T);
+          const int b = mdiv<S::MDIV>(ri, p.m_T, p.T), grow = b * p.Mqp + (ri - b * p.T);
 #pragma unroll
           for (int q = 0; q < NP; ++q) x[k][q] = as_f4(bload(rh, fpiece(grow, 4 * (c.lane + 64 * q), c.RT), 0));
           xc[k] = xcur[(long long)ri * p.A + min(c.lane, p.A - 1)];
@@ -3450,7 +3470,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
         for (int k = 0; k < R; ++k) {
           const int ri = min(r0 + NWAVES * k, r_hi - 1);
           const float rs = rsqrtf(ss[k] * (1.0f / (float)S::H) + (S::YS ? p.eps_final : p.eps));
-          const float* ml = tail_mods_lds(c, ri / p.T);
+          const float* ml = tail_mods_lds(c, mdiv<S::MDIV>(ri, p.m_T, p.T));
 #pragma unroll
           for (int q = 0; q < NP; ++q) {
             const int col = 4 * (c.lane + 64 * q);
@@ -3501,7 +3521,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
       }
     } else if (inproj) {
       for (int it = c.tid; it < nrows * adim; it += NTHREADS) {
-        const int ri = it / adim, a = it - ri * adim;
+        const int ri = mdiv<S::MDIV>(it, p.m_adim, adim), a = it - ri * adim;
         xp[it] = xcur[(long long)ri * p.A + a];
       }
     }
@@ -3523,7 +3543,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
 #pragma unroll
           for (int k = 0; k < IB; ++k) {
             const int row = min(row1 + k * (NTHREADS / 8), p.NRP - 1);
-            const int b = row / p.Mqp, i = row - b * p.Mqp;
+            const int b = mdiv<S::MDIV>(row, p.m_mqp, p.Mqp), i = row - b * p.Mqp;
             sc[k] = ldf4(c.modrow(min(b, p.B - 1), sn) + col);  // layer 0 self-attention AdaRMS scale
             const int ir = min(max(i - p.T, 0), max(p.R - 1, 0));  // (a valid register row, used for register rows only)
             rg[k] = p.R > 0 ? *reinterpret_cast<const uint2*>(p.reg_tok + (long long)ir * S::H + col) : uint2{0u, 0u};
@@ -3532,7 +3552,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
           for (int k = 0; k < IB; ++k) {
             const int row = row1 + k * (NTHREADS / 8);
             if (row >= p.NRP) break;
-            const int b = row / p.Mqp, i = row - b * p.Mqp;
+            const int b = mdiv<S::MDIV>(row, p.m_mqp, p.Mqp), i = row - b * p.Mqp;
             f32x4 v = {0.f, 0.f, 0.f, 0.f};
             if (b < p.B && i < p.T) {
               v = bv0;
@@ -3554,7 +3574,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
         // item: row, 4-column piece q of the task's tiles 2 t (q < 4) and 2 t + 1
         for (int it = c.tid; it < p.NRP * 8; it += NTHREADS) {
           const int row = it >> 3, q = it & 7;
-          const int b = row / p.Mqp, i = row - b * p.Mqp;
+          const int b = mdiv<S::MDIV>(row, p.m_mqp, p.Mqp), i = row - b * p.Mqp;
           const int col = t * 32 + 4 * q;
           f32x4 v, sc;
           uint2 rg;
@@ -3654,7 +3674,7 @@ __device__ __forceinline__ void prefetch_body(Ctx<S>& c, const Desc& d, const in
     // split tasks only store partial sums)
     if constexpr (S::RW) {
       // one 16-column tile per gated-residual task and per reducer (Params::tpr = 1): its slices only
-      if (d.kind == K_RES && t < d.ntask) dma_mods_tile(c, d, t % d.tiles);
+      if (d.kind == K_RES && t < d.ntask) dma_mods_tile(c, d, t - mdiv<S::MDIV>(t, d.m_tiles, d.tiles) * d.tiles);
       else if (d.kind == K_SPLIT && task_first(c, PL_RED) < p.nred) dma_mods_tile(c, d, task_first(c, PL_RED) % S::HT);
     } else if ((d.kind == K_RES && t < d.ntask) || (d.kind == K_SPLIT && task_first(c, PL_RED) < p.nred)) {
       for (int b = 0; b < p.B; ++b) {

@@ -43,8 +43,8 @@ constexpr int MAX_ROWS_PADDED = 512;
 constexpr bool mdiv_exact(int d, int x_max) {
   const uint32_t m = mdiv_m(d);
   for (int x = d; x <= x_max + d; x += d)
-    if (mdiv<true>(x - 1, m, d) != x / d - 1 || mdiv<true>(x, m, d) != x / d) return false;
-  return mdiv<true>(0, m, d) == 0;
+    if (mdiv(x - 1, m) != x / d - 1 || mdiv(x, m) != x / d) return false;
+  return mdiv(0, m) == 0;
 }
 constexpr bool mdiv_exact_upto(int d_max, int x_max, bool times_d) {
   for (int d = 1; d <= d_max; ++d)

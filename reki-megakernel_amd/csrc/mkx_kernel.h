@@ -119,11 +119,10 @@ typedef const __attribute__((address_space(4))) Params CP;
 
 __host__ __device__ constexpr int ceil_to(int a, int m) { return (a + m - 1) / m * m; }
 
-// x / d, x >= 0: by the multiplier m = mdiv_m(d) (ON; exact while x d < 2^20 and x m < 2^32, far above a launch's
-// rows, tiles and tasks), or by dividing
+// x / d, x >= 0, by the multiplier m = mdiv_m(d): exact while x d < 2^20 and x m < 2^32, far above a launch's rows, tiles
+// and tasks
 __host__ __device__ constexpr uint32_t mdiv_m(int d) { return (1u << 20) / (uint32_t)(d > 0 ? d : 1) + 1; }
-template <bool ON>
-__host__ __device__ constexpr int mdiv(int x, uint32_t m, int d) { return ON ? (int)(((uint32_t)x * m) >> 20) : x / d; }
+__host__ __device__ constexpr int mdiv(int x, uint32_t m) { return (int)(((uint32_t)x * m) >> 20); }
 
 template <int H_, int I_, bool W8_ = false, bool RW_ = false, bool YS_ = false, bool PR_ = false, bool LS_ = false>
 struct Shape {
@@ -142,8 +141,8 @@ struct Shape {
   // instructions each. In the row-wise form nearly every workgroup runs every GEMM stage, so this work lies between one
   // task's end and the next one's poll: with the shift fragments' loads ahead of the poll D 6.74 -> 6.48, D-b4 11.79 ->
   // 11.46, B's ten steps 6.30 -> 6.12 ms (the loads alone: 6.66, 11.86 and 6.27). In the form with passes, whose
-  // transitions are off the critical path, it measured 2.70 -> 2.72 ms and more; the attention stages' task order by
-  // multipliers made B 2 % slower.
+  // transitions are off the critical path, it measured 2.70 -> 2.72 ms and more, so its instructions stay as they were;
+  // the attention stages' task order by multipliers made B 2 % slower.
   static constexpr bool MDIV = RW_;
   // CA_LATE: cross-attention DMAs its source K/V after its ready-epoch poll and query rows: the fp16 row-wise
   // instantiations and the two-tile ones (not the other fp8 row-wise ones, whose launches, workload D, measured
@@ -306,7 +305,7 @@ struct Ctx {
     return p.mods + (long long)b * p.mods_sb + (long long)(p.mod_row0 + s) * p.mods_ss;
   }
   __device__ int sample_of(int grow) const {
-    int b = mdiv<S::MDIV>(grow, p.m_mqp, p.Mqp);
+    int b = (S::MDIV ? mdiv(grow, p.m_mqp) : grow / p.Mqp);
     return b < p.B ? b : p.B - 1;
   }
 };
@@ -469,7 +468,7 @@ __device__ __forceinline__ int task_first(Ctx<S>& c, int k) {
 
 // row group (of rgs over the RT row tiles, group g covering [g RT / rgs, (g + 1) RT / rgs)) holding row tile rt
 template <class S>
-__device__ __forceinline__ int row_group_of(Ctx<S>& c, int rt, int rgs) { return mdiv<S::MDIV>((rt + 1) * rgs - 1, c.p.m_RT, c.RT); }
+__device__ __forceinline__ int row_group_of(Ctx<S>& c, int rt, int rgs) { return (S::MDIV ? mdiv((rt + 1) * rgs - 1, c.p.m_RT) : ((rt + 1) * rgs - 1) / c.RT); }
 
 // ------------------------------------------------------------------------------------------------
 // Stage descriptor: what one stage computes, where its operands live, and what to prefetch for it.
@@ -521,7 +520,7 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
   d.sc = nullptr; d.sc2 = nullptr;
   d.yout = nullptr; d.ssout = nullptr; d.ssin = nullptr; d.shs = nullptr;
   d.ntask = 0; d.tiles = 1; d.kind = K_QKV; d.nt = 1; d.mod_off = 0; d.mod_off2 = 0; d.rgs = 1; d.pk = PL_TIN;
-  d.m_tiles = d.m_rgs = mdiv_m(1);
+  if constexpr (S::MDIV) d.m_tiles = d.m_rgs = mdiv_m(1);
   if (q.g == 0) { d.st = ST_TAIL; d.s = 0; d.l = 0; return d; }
   d.s = q.s;
   if (q.l == p.L) {
@@ -543,7 +542,8 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
       if (S::W8) d.sc = p.sc_qkv + (long long)l * 3 * S::H;
       d.out = (float*)(fr + S::qs_off(NRP)); d.yout = (float*)(fr + S::ks_off(NRP)); d.part = (float*)(fr + S::vtb_off(NRP));
       d.ssout = (float*)(fr + S::ssqk_off(NRP)); d.tiles = 6 * S::NH; d.nt = 2; d.shs = shs;
-      d.rgs = p.rgs_qkv; d.pk = PL_QKV; d.m_tiles = mdiv_m(6 * S::NH); d.m_rgs = p.m_rgs_qkv;
+      d.rgs = p.rgs_qkv; d.pk = PL_QKV;
+      if constexpr (S::MDIV) { d.m_tiles = mdiv_m(6 * S::NH); d.m_rgs = p.m_rgs_qkv; }
       break;
     case ST_O:
       d.w = p.wo + l * p.s_o; d.a = (const float*)(fr + S::ysa_off(NRP)); d.out = (float*)(fr + S::h2_off(NRP));
@@ -551,7 +551,8 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
       d.yout = (float*)(fr + S::y2_off(NRP)); d.ssout = (float*)(fr + S::ss2_off(NRP));
       d.res = c.h_in(d.s, l); d.kind = K_RES; d.mod_off = m_sa + 2 * S::H; d.mod_off2 = m_ca;
       d.nt = p.nt_o; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.wstride = (long long)d.nt * S::NKB * S::CH;
-      d.m_tiles = mdiv_m(S::HT); d.rgs = p.rgs_o; d.m_rgs = p.m_rgs_o; d.pk = PL_O;
+      d.rgs = p.rgs_o; d.pk = PL_O;
+      if constexpr (S::MDIV) { d.m_tiles = mdiv_m(S::HT); d.m_rgs = p.m_rgs_o; }
       break;
     case ST_CAO:
       d.w = p.woca + l * p.s_o; d.a = (const float*)(fr + S::yca_off(NRP)); d.out = (float*)(fr + S::h3_off(NRP));
@@ -560,20 +561,23 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
       d.res = (const float*)(fr + S::h2_off(NRP)); d.kind = K_RES;
       d.mod_off = m_ca + 2 * S::H; d.mod_off2 = m_mlp;
       d.nt = p.nt_cao; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.wstride = (long long)d.nt * S::NKB * S::CH;
-      d.m_tiles = mdiv_m(S::HT); d.rgs = p.rgs_cao; d.m_rgs = p.m_rgs_cao; d.pk = PL_CAO;
+      d.rgs = p.rgs_cao; d.pk = PL_CAO;
+      if constexpr (S::MDIV) { d.m_tiles = mdiv_m(S::HT); d.m_rgs = p.m_rgs_cao; }
       break;
     case ST_GU:
       d.w = p.wgu + l * p.s_gu; d.wstride = 2LL * S::NKB * S::CH; d.a = (const float*)(fr + S::y3_off(NRP));
       if (S::W8) { d.sc = p.sc_g + (long long)l * S::I; d.sc2 = p.sc_u + (long long)l * S::I; }
       d.ssin = (const float*)(fr + S::ss3_off(NRP)); d.out = (float*)(fr + S::g_off(NRP));
-      d.tiles = S::IT; d.m_tiles = mdiv_m(S::IT); d.kind = K_GU; d.nt = 2; d.shs = shs + 2 * p.B * S::H * 4; d.pk = PL_GU;
+      d.tiles = S::IT; d.kind = K_GU; d.nt = 2; d.shs = shs + 2 * p.B * S::H * 4; d.pk = PL_GU;
+      if constexpr (S::MDIV) d.m_tiles = mdiv_m(S::IT);
       break;
     case ST_DOWN:
       d.w = p.wd + l * p.s_d; d.a = (const float*)(fr + S::g_off(NRP)); d.out = (float*)(fr + S::hl_off(NRP));
       if (S::W8) d.sc = p.sc_d + (long long)l * S::H;
       d.yout = (float*)(fr + S::yl_off(NRP)); d.ssout = (float*)(fr + S::ssl_off(NRP));
       d.res = (const float*)(fr + S::h3_off(NRP)); d.part = (float*)(fr + S::part_off(NRP));
-      d.nt = p.nt_down; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.m_tiles = mdiv_m(S::HT); d.rgs = S::SK; d.kind = K_SPLIT; d.pk = PL_DOWN;
+      d.nt = p.nt_down; d.tiles = S::RW ? S::HT : S::HT / d.nt; d.rgs = S::SK; d.kind = K_SPLIT; d.pk = PL_DOWN;
+      if constexpr (S::MDIV) d.m_tiles = mdiv_m(S::HT);
       d.mod_off = m_mlp + 2 * S::H; d.mod_off2 = m_next;
       break;
     case ST_SA:
@@ -593,7 +597,7 @@ __device__ __forceinline__ Desc describe(Ctx<S>& c, const StagePos& q) {
 // down projection's splits are packed [tile][split][k-block], so its tiles are nt runs)
 template <class S>
 __device__ __forceinline__ void dma_task_w(Ctx<S>& c, const Desc& d, int t, char* dst) {
-  const int split = mdiv<S::MDIV>(t, d.m_tiles, d.tiles), tile = S::MDIV ? t - split * d.tiles : t % d.tiles;
+  const int tile = S::MDIV ? t - mdiv(t, d.m_tiles) * d.tiles : t % d.tiles, split = S::MDIV ? mdiv(t, d.m_tiles) : t / d.tiles;
   if (d.kind == K_SPLIT) {
     for (int j = 0; j < d.nt; ++j)
       dma_w(c, dst + j * S::NKB * S::CH, d.w + ((long long)(tile * d.nt + j) * S::SK + split) * S::NKB * S::CH,
@@ -910,8 +914,11 @@ __device__ __forceinline__ void gemm_wait(Ctx<S>& c, const Desc& d, BarCtx& bc, 
   } else if (d.st == ST_O || d.st == ST_CAO) {
     flag_wait(bc, d.st == ST_O ? F_SA : F_CA, (rt_hi - rt_lo) * S::NH, [&](int i) {
       const int rt = rt_lo + i / S::NH, hd = i % S::NH;
-      const int sm = mdiv<S::MDIV>(rt, c.p.m_nqt, NQT);
-      return (sm * S::NH + hd) * NQT + (S::MDIV ? rt - sm * NQT : rt % NQT);
+      if constexpr (S::MDIV) {
+        const int sm = mdiv(rt, c.p.m_nqt);
+        return (sm * S::NH + hd) * NQT + rt - sm * NQT;
+      }
+      return ((rt / NQT) * S::NH + hd) * NQT + rt % NQT;
     }, (unsigned long long)g);
   } else if (d.st == ST_GU) {
     flag_wait(bc, F_CAO, (S::RW ? S::HT : S::HT / c.p.nt_cao) * c.p.rgs_cao, [](int i) { return i; }, (unsigned long long)g);
@@ -935,15 +942,15 @@ __device__ __forceinline__ void down_reduce(Ctx<S>& c, const Desc& d, BarCtx& bc
   if constexpr (S::RW) {
     const int rgr = r / S::HT;
     t0 = (r % S::HT) * tpr;
-    rlo = mdiv<S::MDIV>(rgr * RT, c.p.m_rgs_qkv, c.p.nrg);  // (nrg: the QKV stage's row groups)
-    nrt = mdiv<S::MDIV>((rgr + 1) * RT, c.p.m_rgs_qkv, c.p.nrg) - rlo;
+    rlo = mdiv(rgr * RT, c.p.m_rgs_qkv);  // (nrg: the QKV stage's row groups)
+    nrt = mdiv((rgr + 1) * RT, c.p.m_rgs_qkv) - rlo;
   } else {
     t0 = r * tpr;
     rlo = 0;
     nrt = RT;
   }
   // the tile groups (split tasks per split) holding tiles t0 .. t0 + tpr - 1
-  const int nt = S::RW ? 1 : d.nt, g0 = t0 / nt, ng = (t0 + tpr - 1) / nt - g0 + 1;
+  const int g0 = S::RW ? t0 : t0 / d.nt, ng = S::RW ? tpr : (t0 + tpr - 1) / d.nt - g0 + 1;
   flag_wait<1>(bc, F_DPART, S::SK * ng, [&](int i) { return (i % S::SK) * d.tiles + g0 + i / S::SK; }, (unsigned long long)g);
   wait_vm0();  // the staged gate and next AdaRMS scale (the prefetch's DMA) have landed
   __syncthreads();
@@ -1365,7 +1372,7 @@ __device__ __forceinline__ void gemm_stage_rows(Ctx<S>& c, const Desc& d, BarCtx
   const bool ada = d.kind == K_QKV || d.kind == K_GU;
   const int t0 = task_first(c, d.pk);
   for (int t = t0; t < d.ntask; t += c.G) {
-    const int split = mdiv<S::MDIV>(t, d.m_tiles, d.tiles), tile = t - split * d.tiles;
+    const int split = mdiv(t, d.m_tiles), tile = t - split * d.tiles;
     const int qkind = d.kind == K_QKV ? tile / (2 * S::NH) : 0, qhd = (tile >> 1) % S::NH, qj = tile & 1;
     if (t != t0) {
       wait_vm0();
@@ -1374,8 +1381,8 @@ __device__ __forceinline__ void gemm_stage_rows(Ctx<S>& c, const Desc& d, BarCtx
       if (d.kind == K_RES) dma_mods_tile(c, d, tile);
     }
     const int kb0 = d.kind == K_SPLIT ? split * NKB : 0;
-    const int rt_lo = d.kind == K_SPLIT ? 0 : mdiv<S::MDIV>(split * RT, d.m_rgs, d.rgs);
-    const int rt_hi = d.kind == K_SPLIT ? RT : mdiv<S::MDIV>((split + 1) * RT, d.m_rgs, d.rgs);
+    const int rt_lo = d.kind == K_SPLIT ? 0 : mdiv(split * RT, d.m_rgs);
+    const int rt_hi = d.kind == K_SPLIT ? RT : mdiv((split + 1) * RT, d.m_rgs);
     // AdaRMS tasks: the fp16 shift fragments of this wave's k-blocks (lane l: sample l % 16, zeros for the
     // samples >= B), loaded ahead of the poll, so that they land while the task waits
     f16x8 shv[KPW];
@@ -3424,7 +3431,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
     if (!d.first && S::RW && inproj) {
       const float* xn = c.xstep(d.s + 1);
       for (int it = c.tid; it < nrows * adim; it += NTHREADS) {
-        const int ri = mdiv<S::MDIV>(it, p.m_adim, adim), a = it - ri * adim;
+        const int ri = (S::MDIV ? mdiv(it, p.m_adim) : it / adim), a = it - ri * adim;
         xp[it] = xn[(long long)ri * p.A + a];
       }
     } else if (!d.first) {
@@ -3436,9 +3443,11 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
       if constexpr (S::RW) {
         const int ndg = (p.A + TAIL_DG - 1) / TAIL_DG;
         a_lo = inproj ? 0 : (a_out % ndg) * TAIL_DG;
-        a_hi = inproj ? adim : min(a_lo + TAIL_DG, p.A);
+        // only the launch's last x has padded dims that anything reads: the next step takes the real ones (B's ten steps
+        // 6.12 -> 6.07, D 6.48 -> 6.46 ms)
+        a_hi = min(a_lo + TAIL_DG, d.last ? p.A : adim);
         r_lo = (a_out / ndg) * TAIL_RCH;
-        r_hi = min(r_lo + TAIL_RCH, nrows);
+        r_hi = a_lo < a_hi ? min(r_lo + TAIL_RCH, nrows) : r_lo;
       } else {
         a_lo = inproj ? 0 : a_out * TAIL_AC;
         a_hi = inproj ? adim : min(a_lo + TAIL_AC, p.A);
@@ -3453,7 +3462,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
 #pragma unroll
         for (int k = 0; k < R; ++k) {
           const int ri = min(r0 + NWAVES * k, r_hi - 1);
-          const int b = mdiv<S::MDIV>(ri, p.m_T, p.T), grow = b * p.Mqp + (ri - b * p.T);
+          const int b = (S::MDIV ? mdiv(ri, p.m_T) : ri / p.T), grow = b * p.Mqp + (ri - b * p.T);
 #pragma unroll
           for (int q = 0; q < NP; ++q) x[k][q] = as_f4(bload(rh, fpiece(grow, 4 * (c.lane + 64 * q), c.RT), 0));
           xc[k] = xcur[(long long)ri * p.A + min(c.lane, p.A - 1)];
@@ -3470,7 +3479,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
         for (int k = 0; k < R; ++k) {
           const int ri = min(r0 + NWAVES * k, r_hi - 1);
           const float rs = rsqrtf(ss[k] * (1.0f / (float)S::H) + (S::YS ? p.eps_final : p.eps));
-          const float* ml = tail_mods_lds(c, mdiv<S::MDIV>(ri, p.m_T, p.T));
+          const float* ml = tail_mods_lds(c, (S::MDIV ? mdiv(ri, p.m_T) : ri / p.T));
 #pragma unroll
           for (int q = 0; q < NP; ++q) {
             const int col = 4 * (c.lane + 64 * q);
@@ -3521,7 +3530,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
       }
     } else if (inproj) {
       for (int it = c.tid; it < nrows * adim; it += NTHREADS) {
-        const int ri = mdiv<S::MDIV>(it, p.m_adim, adim), a = it - ri * adim;
+        const int ri = (S::MDIV ? mdiv(it, p.m_adim) : it / adim), a = it - ri * adim;
         xp[it] = xcur[(long long)ri * p.A + a];
       }
     }
@@ -3543,7 +3552,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
 #pragma unroll
           for (int k = 0; k < IB; ++k) {
             const int row = min(row1 + k * (NTHREADS / 8), p.NRP - 1);
-            const int b = mdiv<S::MDIV>(row, p.m_mqp, p.Mqp), i = row - b * p.Mqp;
+            const int b = (S::MDIV ? mdiv(row, p.m_mqp) : row / p.Mqp), i = row - b * p.Mqp;
             sc[k] = ldf4(c.modrow(min(b, p.B - 1), sn) + col);  // layer 0 self-attention AdaRMS scale
             const int ir = min(max(i - p.T, 0), max(p.R - 1, 0));  // (a valid register row, used for register rows only)
             rg[k] = p.R > 0 ? *reinterpret_cast<const uint2*>(p.reg_tok + (long long)ir * S::H + col) : uint2{0u, 0u};
@@ -3552,7 +3561,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
           for (int k = 0; k < IB; ++k) {
             const int row = row1 + k * (NTHREADS / 8);
             if (row >= p.NRP) break;
-            const int b = mdiv<S::MDIV>(row, p.m_mqp, p.Mqp), i = row - b * p.Mqp;
+            const int b = (S::MDIV ? mdiv(row, p.m_mqp) : row / p.Mqp), i = row - b * p.Mqp;
             f32x4 v = {0.f, 0.f, 0.f, 0.f};
             if (b < p.B && i < p.T) {
               v = bv0;
@@ -3574,7 +3583,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
         // item: row, 4-column piece q of the task's tiles 2 t (q < 4) and 2 t + 1
         for (int it = c.tid; it < p.NRP * 8; it += NTHREADS) {
           const int row = it >> 3, q = it & 7;
-          const int b = mdiv<S::MDIV>(row, p.m_mqp, p.Mqp), i = row - b * p.Mqp;
+          const int b = (S::MDIV ? mdiv(row, p.m_mqp) : row / p.Mqp), i = row - b * p.Mqp;
           const int col = t * 32 + 4 * q;
           f32x4 v, sc;
           uint2 rg;
@@ -3674,7 +3683,7 @@ __device__ __forceinline__ void prefetch_body(Ctx<S>& c, const Desc& d, const in
     // split tasks only store partial sums)
     if constexpr (S::RW) {
       // one 16-column tile per gated-residual task and per reducer (Params::tpr = 1): its slices only
-      if (d.kind == K_RES && t < d.ntask) dma_mods_tile(c, d, t - mdiv<S::MDIV>(t, d.m_tiles, d.tiles) * d.tiles);
+      if (d.kind == K_RES && t < d.ntask) dma_mods_tile(c, d, t - mdiv(t, d.m_tiles) * d.tiles);
       else if (d.kind == K_SPLIT && task_first(c, PL_RED) < p.nred) dma_mods_tile(c, d, task_first(c, PL_RED) % S::HT);
     } else if ((d.kind == K_RES && t < d.ntask) || (d.kind == K_SPLIT && task_first(c, PL_RED) < p.nred)) {
       for (int b = 0; b < p.B; ++b) {

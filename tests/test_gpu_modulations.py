@@ -1,6 +1,7 @@
 """GPU: ``mkx_modulations`` (through the C ABI, via mkx.modulations.ModulationProjection) against the CPU
 oracle's ``step_modulations`` on the same input c, and the expert run on the kernel's modulation rows.
 Tolerance: fp32 products from split-bf16 operands and a hardware exp in SiLU, |delta| <= 1e-4 max|mods|."""
+import ctypes
 import json
 from dataclasses import replace
 
@@ -8,7 +9,7 @@ import pytest
 import torch
 
 from _cases import TINY, diff, make_case, oracle_dims, oracle_steps
-from mkx import ExpertMegakernel, synthetic as SY
+from mkx import ExpertMegakernel, _lib, synthetic as SY
 from mkx.modulations import ModulationProjection, StepModulations
 from oracle import expert_ref as ER
 
@@ -187,9 +188,23 @@ def test_modulations_row_and_column_edges(R, K, N, fragment_order):
     assert bool(((out - ref).abs() <= bound).all()), float(((out - ref).abs() / S).max())
 
 
+def _input_single_launch(step, N, sc):
+    """mkx_modulation_input, the entry without a workspace, on the weights of a StepModulations."""
+    sc = sc.cuda()
+    out = torch.empty(sc.shape[0], N, step.H, device="cuda")
+    a = _lib.MkxModinArgs(N=N, B=sc.shape[0], H=step.H, tdim=step.tdim, t1_w=step.t1_w.data_ptr(), t1_b=step.t1_b.data_ptr(),
+                          t2_w=step.t2_w.data_ptr(), t2_b=step.t2_b.data_ptr(), state_cond=sc.data_ptr(), sc_stride=step.H,
+                          out=out.data_ptr(), out_stride_b=N * step.H, out_stride_k=step.H)
+    _lib.check(_lib.lib().mkx_modulation_input(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
+               "mkx_modulation_input")
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("workspace", [True, False])
 @pytest.mark.parametrize("N, B, H, tdim", [(1, 1, 256, 32), (10, 1, 768, 256), (15, 5, 512, 64), (16, 2, 768, 160), (17, 3, 1024, 512),
                                            (33, 6, 1024, 96)])
-def test_modulation_input_step_and_width_edges(N, B, H, tdim):
+def test_modulation_input_step_and_width_edges(N, B, H, tdim, workspace):
     """Steps below, at and past a row tile of 16, every width, odd k-block counts of the embedding and more samples than
     waves share a column tile. Against 64 bits, with the error carried through: embedding rounded to fp32 (2^-24), sums of
     n fp32 additions (n 2^-24 of the sum of magnitudes), silu (slope at most 1.1; hardware exp 2^-20)."""
@@ -197,7 +212,7 @@ def test_modulation_input_step_and_width_edges(N, B, H, tdim):
     t1w, t2w = _rand(H, tdim, seed=1, std=0.05).to(bf), _rand(H, H, seed=2, std=0.05).to(bf)
     t1b, t2b, sc = _rand(H, seed=3, std=0.1), _rand(H, seed=4, std=0.1), _rand(B, H, seed=5)
     step = StepModulations(t1w.cuda(), t1b.cuda(), t2w.cuda(), t2b.cuda(), _rand(16, H, seed=6).to(bf).cuda(), _rand(16, seed=7).cuda())
-    out = step.input(N, sc.cuda()).cpu().double()
+    out = (step.input(N, sc.cuda()) if workspace else _input_single_launch(step, N, sc)).cpu().double()
     d = torch.float64
     half = tdim // 2
     arg = 1000.0 * (1.0 - torch.arange(N, dtype=d) / N)[:, None] * 10000.0 ** (-torch.arange(half, dtype=d) / half)

@@ -200,7 +200,7 @@ def probe_bench(reps: int) -> int:
 
 def expert_call_bench(cfg, n: int, name: str) -> int:
     """Times one whole expert call as a policy step runs it, on this library's kernels: the step
-    modulations (mkx_modulation_input: timestep embedding and the small MLP; mkx_modulations: the MODW-wide
+    modulations (mkx_modulation_input_ws: timestep embedding and the small MLP; mkx_modulations: the MODW-wide
     projection), the cross-attention source caches (mkx_source_run), Euler steps 1..N in one launch (run_all)
     and the register-memory append (mkx_ring_append); beside it the same call with the modulations and
     source caches in PyTorch and step 1 as its own launch (the reference's split, src/mk_expert.py:527-533)."""

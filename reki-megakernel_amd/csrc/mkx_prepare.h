@@ -231,7 +231,7 @@ __device__ __forceinline__ void prep_unit(const PrepUnit& q, const SourceParams&
 // groups' workgroups share the stores of them. At most 5 row tiles, so that two workgroups share a CU (256 registers a
 // wave) and one's first loads and epilogue run beside the other's MFMAs.
 // Measured (10 layers, 12 heads, C 2048): one call of 300 rows 44.4 -> 30.9 us (616 TFLOP/s; a large matrix product
-// reaches 1115), eight of 300 down to 41 rows 183.6 -> 121 us, of which the numbering of the valid rows gives the
+// reaches 1115), eight of 300 down to 41 rows 183.6 -> 125 us, of which the numbering of the valid rows gives the
 // larger part. Bound by the operands' way from L2 (25 bytes per cycle and CU at 281 cycles of latency).
 template <int NRT>
 __global__ __launch_bounds__(PREP_BLOCK, 2) void prepare_source_kernel(SourceParams a) {

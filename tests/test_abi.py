@@ -153,6 +153,18 @@ def test_modulation_input_rejects_bad_arguments_without_launching():
     assert L.mkx_modulation_input(ctypes.byref(a), None) == _lib.EINVAL
 
 
+def test_modulation_input_with_workspace_rejects_bad_arguments_without_launching():
+    L = _lib.lib()
+    assert L.mkx_modulation_input_ws(None, None, None) == _lib.EINVAL
+    a = _lib.MkxModinArgs(N=10, B=1, H=640, tdim=256, sc_stride=768, out_stride_b=7680, out_stride_k=768)
+    assert L.mkx_modulation_input_ws(ctypes.byref(a), None, None) == _lib.EUNSUPPORTED
+    a.H = 768
+    for n in ("t1_w", "t1_b", "t2_w", "t2_b", "state_cond", "out"):
+        setattr(a, n, 4096)
+    assert L.mkx_modulation_input_ws(ctypes.byref(a), None, None) == _lib.EINVAL  # no workspace
+    assert L.mkx_modulation_input_ws(ctypes.byref(a), ctypes.c_void_p(4100), None) == _lib.EINVAL  # misaligned
+
+
 def test_query_keys_match_the_header():
     """mkx_query_key values in include/mkx.h equal the binding's constants (a drifted key would query
     something else without any error)."""

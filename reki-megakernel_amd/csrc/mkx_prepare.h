@@ -275,18 +275,19 @@ __global__ __launch_bounds__(PREP_BLOCK, 2) void prepare_source_kernel(SourcePar
   if (g0 * 16 >= nv) return;
   // fragments of k-block kb: context row tile r at (kb NRT + r) KB of the row group, weight column tile j at
   // (kb 4 + j % 4) KB of head j / 4 (an odd head count's last pair repeats its head, never stored)
-  const __amdgpu_buffer_rsrc_t rx = rsrc(a.ctxp + (int64_t)rg * T * NRT * 512);
-  const bf16_t* wsrc = (is_v ? a.wvp : a.wkp) + (int64_t)(l * NH + 2 * pair) * T * 2048;
-  const __amdgpu_buffer_rsrc_t rw0 = rsrc(wsrc), rw1 = rsrc(2 * pair + 1 < NH ? wsrc + (int64_t)T * 2048 : wsrc);
+  // (64-bit k-block offsets: a context of 2^25 columns has 4 GB of weights per head)
   const uint32_t vl = (uint32_t)lane * 16;
+  const char* const xsrc = (const char*)(a.ctxp + (int64_t)rg * T * NRT * 512);
+  const char* const wsrc0 = (const char*)((is_v ? a.wvp : a.wkp) + (int64_t)(l * NH + 2 * pair) * T * 2048);
+  const char* const wsrc1 = 2 * pair + 1 < NH ? wsrc0 + (int64_t)T * 4096 : wsrc0;
   const int nk = (T - wave + 3) / 4;  // this wave's k-blocks (0 where T < 4 leaves it none)
   auto ldw = [&](int i, int j) {  // (past the last k-block: that one again, unused)
-    const int kb = wave + 4 * max(min(i, nk - 1), 0);
-    return bload(j < 4 ? rw0 : rw1, vl + (j & 3) * 1024, (uint32_t)min(kb, T - 1) * 4096);
+    const int kb = min(wave + 4 * max(min(i, nk - 1), 0), T - 1);
+    return bload(rsrc((j < 4 ? wsrc0 : wsrc1) + (int64_t)kb * 4096), vl + (j & 3) * 1024, 0);
   };
   auto ldx = [&](int i, int r) {
-    const int kb = wave + 4 * max(min(i, nk - 1), 0);
-    return bload(rx, vl, (uint32_t)(min(kb, T - 1) * NRT + r) * 1024);
+    const int kb = min(wave + 4 * max(min(i, nk - 1), 0), T - 1);
+    return bload(rsrc(xsrc + (int64_t)kb * NRT * 1024), vl, r * 1024);
   };
   u32x4 xf[NRT], wf[WB][8];
 #pragma unroll

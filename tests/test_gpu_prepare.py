@@ -6,6 +6,7 @@ Tolerance: accumulation order (MFMA vs the CPU's) and rsqrt can move a bf16 roun
 rotation mixes the two halves of a head, so K is bounded per RoPE pair, |delta| <= 2^-6 |(x_d, x_d+32)|,
 and V per element, |delta| <= 2^-7 |v| + 2^-12. A wrong position, sign, norm weight or head fails both by
 orders of magnitude."""
+import ctypes
 import json
 from dataclasses import replace
 
@@ -13,7 +14,7 @@ import pytest
 import torch
 
 from _cases import TINY, diff, make_case, oracle_dims, oracle_steps
-from mkx import ExpertMegakernel, synthetic as SY
+from mkx import ExpertMegakernel, _lib, synthetic as SY
 from mkx.prepare import SourcePrepare
 from oracle import expert_ref as ER
 
@@ -271,3 +272,44 @@ def test_frames_with_ring_append_as_two_graphs_match_eager():
     mk.check()
     assert kss == [max(cfg.PM - (f + 1) * R, 0) for f in range(4)]
     _report("frames as two graphs (A)", frames=4, kv_start=kss)
+
+
+def _source_run(wk, wv, k_norm, ctx, lens, cos, sin, kca, vca, stride):
+    """mkx_source_create and mkx_source_run on caller-made buffers: wk, wv [L, NH * 64, C], kca / vca per-layer addresses,
+    `stride` elements between samples."""
+    L, NH, (B, SP, C) = wk.shape[0], wk.shape[1] // 64, ctx.shape
+    lib, stream = _lib.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    h = ctypes.c_void_p()
+    dims = _lib.MkxSourceDims(L=L, NH=NH, HD=64, C=C, max_rows=B * SP, eps=1e-6)
+    _lib.check(lib.mkx_source_create(ctypes.byref(dims), ctypes.c_void_p(wk.data_ptr()), ctypes.c_void_p(wv.data_ptr()),
+                                     ctypes.c_void_p(k_norm.data_ptr()), stream, ctypes.byref(h)), "mkx_source_create")
+    a = _lib.MkxSourceArgs(B=B, SP=SP, ctx=ctx.data_ptr(), ca_len=lens.data_ptr(), cos=cos.data_ptr(), sin=sin.data_ptr())
+    for l in range(L):
+        a.kca[l], a.vca[l] = kca[l], vca[l]
+    a.src_stride_b = stride
+    _lib.check(lib.mkx_source_run(h, ctypes.byref(a), stream), "mkx_source_run")
+    torch.cuda.synchronize()
+    lib.mkx_source_destroy(h)
+
+
+def test_prepare_context_of_four_gigabytes_of_weights_per_head():
+    """A context so wide that the byte offsets of a head's weights and of a row group's context pass 2^32. Operands are -1, 0
+    and 1, so every partial sum is a whole number below 2^24 and the projections are exact: V is the rounded sum itself."""
+    C, SP = (1 << 25) + 96, 20
+    g = torch.Generator(device="cuda").manual_seed(3)
+    trits = lambda *s: torch.randint(-1, 2, s, generator=g, device="cuda", dtype=torch.int8).bfloat16()  # noqa: E731
+    wk, wv, ctx = trits(1, 64, C), trits(1, 64, C), trits(1, SP, C)
+    out = torch.full((2, SP, 64), float("nan"), dtype=torch.bfloat16, device="cuda")
+    cos, sin = torch.ones(SP, 64, device="cuda"), torch.zeros(SP, 64, device="cuda")
+    _source_run(wk, wv, torch.zeros(1, 64, dtype=torch.bfloat16, device="cuda"), ctx,
+                torch.tensor([SP], dtype=torch.int32, device="cuda"), cos, sin, [out[0].data_ptr()], [out[1].data_ptr()], SP * 64)
+    k, v = torch.zeros(2, SP, 64, dtype=torch.float64, device="cuda")
+    for c in range(0, C, 1 << 20):
+        x = ctx[0, :, c:c + (1 << 20)].double()
+        k += x @ wk[0, :, c:c + (1 << 20)].double().T
+        v += x @ wv[0, :, c:c + (1 << 20)].double().T
+    assert torch.equal(out[1], v.bfloat16())
+    k = k.bfloat16().double()
+    k = k * torch.rsqrt((k * k).mean(-1, keepdim=True) + 1e-6)
+    # one rounding to bf16 (2^-9) of a value known to a few fp32 roundings
+    assert bool(((out[0].double() - k).abs() <= 2.0 ** -8 * k.abs()).all())

@@ -54,6 +54,20 @@ constexpr bool mdiv_exact_upto(int d_max, int x_max, bool times_d) {
 static_assert(mdiv_exact_upto(256, FLAG_MAX, false), "tasks by tiles; rows by a sample's rows or row tiles; row tiles by row groups");
 static_assert(mdiv_exact_upto(24, MAX_ROWS_PADDED, true), "(row, action dim) items by action dims");
 
+// prep_first_above over every sample count: samples of 0, 1 and 2 rows, so that keys repeat
+constexpr bool prep_search_exact(int n_max) {
+  for (int n = 1; n <= n_max; ++n) {
+    auto key = [](int i) { return i + (i + 1) / 3; };
+    for (int v = 0; v < key(n - 1); ++v) {
+      int b = 0;
+      while (v >= key(b)) ++b;
+      if (prep_first_above(v, n, key) != b) return false;
+    }
+  }
+  return true;
+}
+static_assert(prep_search_exact(PREP_MAP_B), "a numbered row's sample");
+
 // W [L][N][K] row-major bf16 -> fp16 chunks (l, t, kb): dst[l*dls + (t'*tstride + toff + kb)*512 + lane*8 + j]
 // = W[l][t*16 + lane%16][kb*32 + 8(lane/16) + j] (the MFMA 16x16x32 operand layout). t' = t, or with
 // `pairs` the 16-column tiles of each 64-column head reordered 0, 2, 1, 3 (a task's d and d + 32 tiles

@@ -45,19 +45,35 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const bf16_t* __restrict
 // more samples number every row, v = b SP + s.
 constexpr int PREP_MAP_B = 64;
 struct PrepRows {
-  int n;   // lane b: valid rows of samples 0 .. b
-  int nv;  // rows numbered
-  __device__ __forceinline__ int end(int b) const { return __builtin_amdgcn_readlane(n, b); }
+  const int* ends;  // LDS, two samples and more: valid rows of samples 0 .. b
+  int nv;           // rows numbered
 };
-__device__ __forceinline__ PrepRows prep_rows(const int32_t* ca_len, int B, int SP) {
-  if (B > PREP_MAP_B) return PrepRows{0, B * SP};
-  const int lane = threadIdx.x & 63;
-  int n = lane < B ? min(max(ca_len[lane], 0), SP) : 0;
-  for (int d = 1; d < B; d *= 2) {
-    const int o = __shfl_up(n, d);
-    if (lane >= d) n += o;
+// The first of n ascending keys that is above v (the last at the latest), by halves. The search runs per lane on LDS: a
+// scan of the samples by lane reads of the prefix sums took as many steps as there are samples (64 samples of 37 rows
+// 244 us a call against 196 with the rows numbered by division) and read lanes that the caller's branch had switched off.
+template <class F>
+__host__ __device__ constexpr int prep_first_above(int v, int n, F key) {
+  int b = 0, d = 1;
+  while (2 * d < n) d *= 2;
+  for (; d > 0; d /= 2)
+    if (b + d < n && v >= key(b + d - 1)) b += d;
+  return b;
+}
+// (every thread of the workgroup calls this once, ahead of any return; `ends` is LDS of the caller's)
+__device__ __forceinline__ PrepRows prep_rows(const int32_t* ca_len, int B, int SP, int (&ends)[PREP_MAP_B]) {
+  if (B > PREP_MAP_B) return PrepRows{ends, B * SP};
+  if (B == 1) return PrepRows{ends, min(max(ca_len[0], 0), SP)};
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    int n = lane < B ? min(max(ca_len[lane], 0), SP) : 0;
+    for (int d = 1; d < B; d *= 2) {
+      const int o = __shfl_up(n, d);
+      if (lane >= d) n += o;
+    }
+    ends[lane] = n;
   }
-  return PrepRows{n, __builtin_amdgcn_readlane(n, B - 1)};
+  __syncthreads();
+  return PrepRows{ends, __builtin_amdgcn_readfirstlane(ends[B - 1])};
 }
 // (sample, source row) of row v < nv
 __device__ __forceinline__ void prep_row_at(int v, int B, int SP, const PrepRows& rows, int& b, int& s) {
@@ -66,13 +82,8 @@ __device__ __forceinline__ void prep_row_at(int v, int B, int SP, const PrepRows
     s = v - b * SP;
     return;
   }
-  b = 0;
-  int start = 0;
-  for (int i = 0; i + 1 < B; ++i) {
-    const int e = rows.end(i);
-    if (v >= e) { b = i + 1; start = e; }
-  }
-  s = v - start;
+  b = prep_first_above(v, B, [&](int i) { return rows.ends[i]; });
+  s = v - (b ? rows.ends[b - 1] : 0);
 }
 
 // The call's context [B, SP, C] into fragment order by row number v: out[g][t][j][lane][8] as pack_rows_kernel,
@@ -81,7 +92,8 @@ __device__ __forceinline__ void prep_row_at(int v, int B, int SP, const PrepRows
 __global__ __launch_bounds__(256) void pack_ctx_kernel(const bf16_t* __restrict__ in, bf16_t* __restrict__ out,
                                                        const int32_t* __restrict__ ca_len, int B, int SP, int C, int S,
                                                        long long n_out) {
-  const PrepRows rows = prep_rows(ca_len, B, SP);
+  __shared__ int ends[PREP_MAP_B];
+  const PrepRows rows = prep_rows(ca_len, B, SP, ends);
   const int nv = rows.nv;
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n_out) return;
@@ -252,7 +264,8 @@ __global__ __launch_bounds__(PREP_BLOCK, 2) void prepare_source_kernel(SourcePar
   const int rg = sb * a.sbw + tix % sw, cgp = tix / sw;
   const int pair = cgp % NP, lk = cgp / NP, l = lk >> 1, is_v = lk & 1;
   bf16_t* const outl = (bf16_t*)(is_v ? a.vca[l] : a.kca[l]);
-  const PrepRows rows = prep_rows(a.ca_len, a.B, a.SP);
+  __shared__ int ends[PREP_MAP_B];
+  const PrepRows rows = prep_rows(a.ca_len, a.B, a.SP, ends);
   const int nv = rows.nv;
   if (a.B <= PREP_MAP_B && nv < a.B * a.SP) {
     // this row group's share of the rows past their sample's length (numbered over the samples), zeroed: 16 bytes
@@ -260,11 +273,9 @@ __global__ __launch_bounds__(PREP_BLOCK, 2) void prepare_source_kernel(SourcePar
     const int nd = a.B * a.SP - nv, d1 = (int)((long long)nd * (rg + 1) / ngr);
     const int tpr = 2 * pair + 1 < NH ? 16 : 8, piece = threadIdx.x % tpr;
     for (int d = (int)((long long)nd * rg / ngr) + (int)threadIdx.x / tpr; d < d1; d += PREP_BLOCK / tpr) {
-      int b = 0, past = 0;  // past: valid rows of the samples before b
-      for (int i = 0; i + 1 < a.B; ++i)
-        if (d >= (i + 1) * a.SP - rows.end(i)) { b = i + 1; past = rows.end(i); }
-      // (the sample's valid rows come first)
-      const int s = d - (b * a.SP - past) + min(max(a.ca_len[b], 0), a.SP);
+      const int b = prep_first_above(d, a.B, [&](int i) { return (i + 1) * a.SP - rows.ends[i]; });
+      const int past = b ? rows.ends[b - 1] : 0, len = (a.B > 1 ? rows.ends[b] : nv) - past;
+      const int s = d - (b * a.SP - past) + len;  // (the sample's valid rows come first)
       bf16_t* o = outl + (int64_t)b * a.src_sb + ((int64_t)s * NH + 2 * pair) * 64 + piece * 8;
       const u32x2 z = {0u, 0u};
       *reinterpret_cast<u32x2*>(o) = z;

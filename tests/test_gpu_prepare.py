@@ -15,7 +15,7 @@ import torch
 
 from _cases import TINY, diff, make_case, oracle_dims, oracle_steps
 from mkx import ExpertMegakernel, _lib, synthetic as SY
-from mkx.prepare import SourcePrepare
+from mkx.prepare import SourcePrepare, rope_table
 from oracle import expert_ref as ER
 
 pytestmark = pytest.mark.gpu
@@ -313,3 +313,48 @@ def test_prepare_context_of_four_gigabytes_of_weights_per_head():
     k = k * torch.rsqrt((k * k).mean(-1, keepdim=True) + 1e-6)
     # one rounding to bf16 (2^-9) of a value known to a few fp32 roundings
     assert bool(((out[0].double() - k).abs() <= 2.0 ** -8 * k.abs()).all())
+
+
+@pytest.mark.parametrize("NH, B, SP, C, lens", [
+    (3, 3, 37, 160, [37, 0, 20]),                  # odd head count: the last head pair is one head wide
+    (1, 5, 31, 96, [0, 31, 0, 17, 0]),             # empty samples first, between and last
+    (4, 2, 100, 64, [0, 0]),                       # no valid row at all
+    (2, 1, 600, 96, [333]),                        # fewer valid rows than row groups launched
+    (3, 64, 5, 64, [(7 * b) % 6 for b in range(64)]),
+    (3, 66, 5, 64, [(7 * b) % 6 for b in range(66)]),  # more samples than are numbered densely
+    (2, 33, 64, 64, [64 - 2 * b for b in range(33)]),
+    (2, 2, 33, 64, [-2, 40]),                      # lengths outside [0, SP]
+])
+def test_prepare_writes_every_row_and_nothing_else(NH, B, SP, C, lens):
+    """Buffers of NaNs with a sample stride past SP * NH * 64 and guards on both sides: rows past a sample's length become
+    exactly 0, the others the result, and the gaps and guards stay as they were. One bf16 rounding may move by a unit, and
+    the rotation mixes the two halves of a head (the module's tolerances)."""
+    L, NAN, G = 2, 0x7FC1, 512
+    row = NH * 64
+    stride = SP * row + 68
+    g = torch.Generator().manual_seed(B)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    wk, wv, kn = (rnd(L, row, C) * 0.1).bfloat16(), (rnd(L, row, C) * 0.1).bfloat16(), (rnd(L, 64) * 0.1).bfloat16()
+    ctx = rnd(B, SP, C).bfloat16()
+    cos, sin = rope_table(SP, device="cpu")
+    buf = torch.full((2, L, G + B * stride + G), NAN, dtype=torch.int16, device="cuda")
+    at = lambda i, l: buf[i, l].data_ptr() + 2 * G  # noqa: E731
+    _source_run(wk.cuda(), wv.cuda(), kn.cuda(), ctx.cuda(), torch.tensor(lens, dtype=torch.int32, device="cuda"), cos.cuda(),
+                sin.cuda(), [at(0, l) for l in range(L)], [at(1, l) for l in range(L)], stride)
+    buf = buf.cpu()
+    body = buf[:, :, G:G + B * stride].view(2, L, B, stride)
+    assert bool((buf[:, :, :G] == NAN).all() and (buf[:, :, G + B * stride:] == NAN).all())
+    assert bool((body[..., SP * row:] == NAN).all())
+    bits = body[..., :SP * row].reshape(2, L, B, SP, NH, 64)
+    dead = torch.arange(SP)[None] >= torch.tensor(lens)[:, None]
+    assert bool((bits[:, :, dead] == 0).all())
+    gk, gv = bits.contiguous().view(torch.bfloat16).double()
+    x, live = ctx.double(), ~dead
+    for l in range(L):
+        v = (x @ wv[l].double().T).bfloat16().double().view(B, SP, NH, 64)
+        k = (x @ wk[l].double().T).bfloat16().double().view(B, SP, NH, 64)
+        n = (k * torch.rsqrt((k * k).mean(-1, keepdim=True) + 1e-6) * (1 + kn[l].double())).bfloat16().double()
+        k = n * cos.double()[:, None] + torch.cat([-n[..., 32:], n[..., :32]], -1) * sin.double()[:, None]
+        pair = torch.sqrt(n[..., :32] ** 2 + n[..., 32:] ** 2).repeat(1, 1, 1, 2)
+        assert bool(((gv[l] - v).abs() <= 2.0 ** -7 * v.abs() + 2.0 ** -12)[live].all())
+        assert bool(((gk[l] - k).abs() <= 2.0 ** -6 * pair + 1e-6)[live].all())

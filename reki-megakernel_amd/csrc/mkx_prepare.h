@@ -337,11 +337,13 @@ __global__ __launch_bounds__(PREP_BLOCK, 2) void prepare_source_kernel(SourcePar
 #pragma unroll
   for (int s = 0; s < WB - 1; ++s)
     if (i0 + s < nk) step(s, i0 + s);
+  // the lane's number anew: kept over the k-loop, the thread index it came from was the one register too many there
+  const int el = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   // the K norm weights of this lane's 16 columns d = 16 j + 4 (lane >> 4) + i (4 bf16 per j)
   uint2 wnv[4];
   if (!is_v) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wnv[j] = *reinterpret_cast<const uint2*>(a.k_norm + l * 64 + 16 * j + 4 * (lane >> 4));
+    for (int j = 0; j < 4; ++j) wnv[j] = *reinterpret_cast<const uint2*>(a.k_norm + l * 64 + 16 * j + 4 * (el >> 4));
   }
   // Units u = (row tile u / 2, head u % 2), PREP_UPP per phase: every wave leaves its part of each in LDS
   // ([unit][wave][column tile][lane]), then each wave sums and stores one of them. Lane: columns d = 16 j + 4 (lane >> 4)
@@ -352,14 +354,14 @@ __global__ __launch_bounds__(PREP_BLOCK, 2) void prepare_source_kernel(SourcePar
     static_assert(PREP_UPP == 4, "one unit per wave and phase");
     const int u = min(u0 + wave, 2 * NRT - 1);  // (a last phase of fewer units repeats one, unstored)
     PrepUnit q;
-    prep_unit_load(q, a, rows, g0 + (u >> 1), is_v, lane);
+    prep_unit_load(q, a, rows, g0 + (u >> 1), is_v, el);
     if (u0) __syncthreads();  // the phase before has been read
 #pragma unroll
     for (int v = u0; v < min(u0 + PREP_UPP, 2 * NRT); ++v)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) pt[(((v - u0) * 4 + wave) * 4 + j) * 64 + lane] = acc[v >> 1][(v & 1) * 4 + j];
+      for (int j = 0; j < 4; ++j) pt[(((v - u0) * 4 + wave) * 4 + j) * 64 + el] = acc[v >> 1][(v & 1) * 4 + j];
     __syncthreads();
-    if (u0 + wave < 2 * NRT) prep_unit(q, a, pt + (u - u0) * 1024, 2 * pair + (u & 1), is_v, outl, wnv, lane);
+    if (u0 + wave < 2 * NRT) prep_unit(q, a, pt + (u - u0) * 1024, 2 * pair + (u & 1), is_v, outl, wnv, el);
   }
 }
 

@@ -256,8 +256,8 @@ int mkx_source_run(mkx_source* h, const mkx_source_args* args, void* stream);
  * loops, harnesses that forbid hipMalloc); no counterpart in the reference. Same arguments, kernels and
  * results as mkx_source_run, but the call's packed context is staged in a static device array of the
  * library (16 MiB per GPU, held until the process ends) instead of the handle's buffer, and the call
- * allocates nothing. A context whose packed form ((ceil32(B * SP) + 160) rows of C * 2 bytes: the rows rounded
- * up to 32 plus 160 rows of padding for the largest workgroup's reads) exceeds 16 MiB is refused with MKX_EINVAL. Every call on one GPU shares that array: calls that overlap on one GPU
+ * allocates nothing. A context whose (ceil32(B * SP) + 160) rows of C * 2 bytes (its rows rounded up to 32, and padding)
+ * exceed 16 MiB is refused with MKX_EINVAL. Every call on one GPU shares that array: calls that overlap on one GPU
  * (concurrent streams, other threads) race and must be serialised by the caller. */
 int mkx_source_run_noalloc(mkx_source* h, const mkx_source_args* args, void* stream);
 int mkx_source_destroy(mkx_source* h);

@@ -854,10 +854,13 @@ int mkx_ring_append(const mkx_ring_args* a, void* stream_) {
 
 }  // extern "C"
 
-// Static staging for mkx_source_run_noalloc: the call's context in fragment order (ceil32(B * SP) + PREP_ROW_PAD
-// rows of C bf16 values, prep_ctx_bytes) lives in this file-scope device array instead of the handle's allocation. Each GPU holds its own copy until the
-// process ends; calls on one GPU share it (the last call's contents stay, and calls that overlap race).
+// Static staging for mkx_source_run_noalloc: the call's context in fragment order lives in this file-scope device array
+// instead of the handle's allocation. Each GPU holds its own copy until the process ends; calls on one GPU share it (the
+// last call's contents stay, and calls that overlap race). Which contexts fit is part of the interface (mkx.h): rows
+// rounded up to 32 plus SOURCE_SCRATCH_PAD, whatever padding the kernel of the day needs.
 constexpr long long SOURCE_SCRATCH_BYTES = 16LL << 20;
+constexpr int SOURCE_SCRATCH_PAD = 160;
+static_assert(SOURCE_SCRATCH_PAD >= PREP_ROW_PAD, "the static scratch covers the kernel's padding");
 static __device__ __align__(256) char scratch[SOURCE_SCRATCH_BYTES];
 
 namespace {
@@ -1056,7 +1059,7 @@ int mkx_source_run(mkx_source* h, const mkx_source_args* a, void* stream_) {
 int mkx_source_run_noalloc(mkx_source* h, const mkx_source_args* a, void* stream_) {
   const int rc = source_args_check(h, a, "mkx_source_run_noalloc");
   if (rc != MKX_OK) return rc;
-  const long long need = prep_ctx_bytes(a->B * a->SP, h->dims.C);
+  const long long need = ((a->B * a->SP + 31LL) / 32 * 32 + SOURCE_SCRATCH_PAD) * h->dims.C * 2;
   if (need > SOURCE_SCRATCH_BYTES)
     return fail(MKX_EINVAL, "mkx_source_run_noalloc: the packed context (" + std::to_string(need) +
                                 " bytes) exceeds the static scratch of " + std::to_string(SOURCE_SCRATCH_BYTES) + " bytes");

@@ -2,6 +2,8 @@
 calls in a row, the second with a smaller context, each equal bit for bit to mkx_source_run on the same
 inputs (the static array keeps the first call's staging, which the second must not read), and a context
 too large for the static array refused before any launch."""
+from dataclasses import replace
+
 import pytest
 import torch
 
@@ -40,4 +42,21 @@ def test_static_scratch_source_preparation_matches_the_allocating_one():
     with pytest.raises(MkxError) as ei:
         prep(too_big, torch.tensor([4100], dtype=torch.int32, device="cuda"), static_scratch=True)
     assert ei.value.status == _lib.EINVAL
+    prep.close()
+
+
+def test_static_scratch_takes_what_the_header_says():
+    """(ceil32(B * SP) + 160) rows of C * 2 bytes in 16 MiB: at C 2048, 3936 rows are the last accepted and 3937 refused."""
+    cfg = replace(SY.WORKLOADS["A"], L=1)
+    prep = SourcePrepare(SY.SyntheticReki(cfg, SY.make_weights(cfg, 0), device="cuda"))
+    g = torch.Generator(device="cuda").manual_seed(6)
+    for B, SP, fits in ((1, 3936, True), (3, 1312, True), (1, 3937, False), (31, 127, False)):
+        ctx = torch.randn(B, SP, 2048, generator=g, device="cuda").to(torch.bfloat16)
+        lens = torch.full((B,), SP, dtype=torch.int32, device="cuda")
+        if fits:
+            assert _same(prep(ctx, lens, static_scratch=True), prep(ctx, lens))
+        else:
+            with pytest.raises(MkxError) as ei:
+                prep(ctx, lens, static_scratch=True)
+            assert ei.value.status == _lib.EINVAL
     prep.close()

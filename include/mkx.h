@@ -266,7 +266,8 @@ int mkx_source_destroy(mkx_source* h);
  * gate of every layer and Euler step of a call in one product (N = MODW = 9 L H + 2 H). Reference: the
  * mods rows the expert reads (src/mk_expert.py:336-340), made by REKI's _step_modulations
  * (mk_expert.py:529: mods, dt = model._step_modulations(num_steps, state_cond)), whose last layer this is.
- * fp32 in and out, bf16 weights; silu(c) is split into bf16 hi + lo MFMA operands. Asynchronous. */
+ * fp32 in and out, bf16 weights; silu(c) is split into three bf16 MFMA operands (as exact as fp32), and a row's result
+ * is the same bits whatever the number of rows. Asynchronous. */
 typedef struct {
   int32_t R;               /* rows: samples x Euler steps */
   int32_t K;               /* input width H: 256, 512, 768 or 1024 */

@@ -944,19 +944,30 @@ int modin_check(const mkx_modin_args* a, const char* who) {
   return MKX_OK;
 }
 
-// The modulation projection of a.R rows: row groups of at most MODP_MAX_NRT row tiles, as even as they come (each
-// group streams the weights once more), one workgroup per CU and group, two per CU where one row tile leaves
-// the registers for it.
+// The modulation projection of a.R rows: row groups of at most modp_max_nrt() row tiles, as even as they come (four tiles of
+// K <= 768 as two groups of two: 64 rows 25.6 us against 28.6 as one), each over every column range. The number of ranges
+// is the largest of those whose rounds of workgroups take the fewest column tiles, a workgroup's start (silu(c) of its rows)
+// counted as MODP_FIXED of them (not counted, 1000 rows take 4 % longer).
+constexpr int MODP_FIXED = 4;
 template <int KT>
 void modproj_launch(const mkx_modproj_args& a, hipStream_t stream) {
-  const int nrt = (a.R + 15) / 16, ngr = (nrt + MODP_MAX_NRT - 1) / MODP_MAX_NRT, per = (nrt + ngr - 1) / ngr;
-  const dim3 grid((unsigned)std::min(a.N / 16, per == 1 ? 2 * MODP_GRID : MODP_GRID), (unsigned)((nrt + per - 1) / per)), block(64 * MODP_WAVES);
+  const int nrt = (a.R + 15) / 16, MAX = nrt == 4 && KT <= 24 ? 2 : modp_max_nrt<KT>();
+  const int ngr0 = (nrt + MAX - 1) / MAX, per = (nrt + ngr0 - 1) / ngr0, ngr = (nrt + per - 1) / per;
+  const int slots = per == 1 ? 2 * MODP_GRID : MODP_GRID, nct = a.N / 16;
+  int y = 1;
+  long long best = -1;
+  for (int i = 1; i * MODP_XCDS <= slots; ++i) {
+    const int nr = i * MODP_XCDS;
+    const long long cost = ((long long)nr * ngr + slots - 1) / slots * ((nct + nr - 1) / nr + MODP_FIXED);
+    if (best < 0 || cost <= best) { best = cost; y = i; }
+  }
+  const dim3 grid((unsigned)(MODP_XCDS * ngr), (unsigned)y), block(64 * MODP_WAVES);
   switch (per) {
     case 1: hipLaunchKernelGGL((modproj_kernel<KT, 1>), grid, block, 0, stream, a); break;
     case 2: hipLaunchKernelGGL((modproj_kernel<KT, 2>), grid, block, 0, stream, a); break;
     case 3: hipLaunchKernelGGL((modproj_kernel<KT, 3>), grid, block, 0, stream, a); break;
     case 4: hipLaunchKernelGGL((modproj_kernel<KT, 4>), grid, block, 0, stream, a); break;
-    default: hipLaunchKernelGGL((modproj_kernel<KT, 5>), grid, block, 0, stream, a); break;
+    default: hipLaunchKernelGGL((modproj_kernel<KT, modp_max_nrt<KT>()>), grid, block, 0, stream, a); break;
   }
 }
 

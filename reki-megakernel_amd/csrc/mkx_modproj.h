@@ -4,9 +4,10 @@
 // REKI's _step_modulations makes them, mk_expert.py:529).
 //
 // HBM-bound on W (bf16 [MODW, H]: 108.5 MB for L10 H768), so each weight byte is read once and the weights are
-// what streams: a workgroup keeps silu(c) of all its rows in registers for the whole launch (each of its 8
-// waves an eighth of K, split into two or three bf16 parts, an MFMA per part and fragment) and walks a contiguous range of 16-column tiles, every wave loading its own K / 8 of a tile's
-// weights several tiles ahead.
+// what streams: a workgroup keeps silu(c) of up to five 16-row tiles on the chip for the whole launch (each of its 8
+// waves an eighth of K, split into three bf16 parts, an MFMA per part and fragment) and walks a contiguous range of
+// 16-column tiles, every wave loading its own K / 8 of a tile's weights a few tiles ahead. The arithmetic of a row, and
+// the order of its sums, are the same whatever the number of rows: its bits do not depend on its company.
 #pragma once
 
 #include "mkx.h"
@@ -15,8 +16,9 @@
 namespace mkx {
 
 constexpr int MODP_WAVES = 8;     // waves of a projection workgroup, each over 1 / 8 of K
-constexpr int MODP_MAX_NRT = 5;   // row tiles of 16 held by a workgroup
-constexpr int MODP_GRID = 256;    // workgroups per row group: one per CU (two with one row tile)
+constexpr int MODP_GRID = 256;    // workgroups at once: one per CU of an MI355X (two with one row tile)
+constexpr int MODP_XCDS = 8;      // XCDs the dispatcher deals consecutive workgroups to
+constexpr int MODP_PARTS = 3;     // bf16 parts of silu(c): as exact as fp32, and the same for every number of rows
 
 typedef float modp_f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 modp_bf16x2 __attribute__((ext_vector_type(2)));
@@ -55,31 +57,41 @@ __device__ __forceinline__ void modp_silu_split(f32x4 x0, f32x4 x1, bf16x8 (&f)[
   for (int i = 0; i < NS; ++i) f[i] = __builtin_bit_cast(bf16x8, o[i]);
 }
 
-// column tiles of weights a wave has in flight ahead of the one it multiplies: KW KB each
+// column tiles of weights a wave has in flight ahead of the one it multiplies, KW KB each. With one row tile two
+// workgroups share a CU, and more in flight is better while 128 registers hold it; with more rows the time goes to the
+// products as well, and two tiles ahead are enough (K 768, 40 rows 25.1 us with four ahead, 23.3 with two; 80 rows 33.9
+// with three, 31.3 with two, 33.5 with one).
 template <int KT, int NRT>
-constexpr int modp_ahead() { return KT <= 8 ? 8 : KT <= 24 ? 4 : NRT == 2 || NRT == 3 ? 4 : 3; }
+constexpr int modp_ahead() { return NRT > 1 ? 2 : KT <= 8 ? 8 : KT <= 24 ? 4 : 3; }
 
-// bf16 parts of silu(c): three where the registers hold them
-template <int NRT>
-constexpr int modp_parts() { return NRT <= 3 ? 3 : 2; }
+// row tiles of 16 that a workgroup holds at most, and the number of them whose third part lies in LDS: what the registers
+// do not hold of the 15 to 20 KB per row tile and wave (K 768, 80 rows: 32.3 us with none in LDS, 31.4 with one tile)
+template <int KT>
+constexpr int modp_max_nrt() { return KT <= 24 ? 5 : 4; }
+template <int KT, int NRT>
+constexpr int modp_lds_tiles() { return KT * NRT > 120 ? 2 : KT * NRT > 100 ? 1 : 0; }
 
-// grid: x = workgroups over contiguous ranges of 16-column tiles, y = groups of NRT row tiles. Wave w holds
-// k-blocks [KW w, KW (w + 1)), KW = KT / 8, of silu(c) of every row of the group (NRT KW fragments in modp_parts() parts) and
-// multiplies them with its KW weight fragments of one column tile after the other; the 8 waves' partial tiles
+// grid: x = MODP_XCDS ranges of 16-column tiles x the groups of NRT row tiles, y = the further ranges; the workgroups of
+// one range lie MODP_XCDS apart, so that one XCD runs them side by side and the weights come from beyond its L2 once. Wave w
+// holds k-blocks [KW w, KW (w + 1)), KW = KT / 8, of silu(c) of every row of the group (NRT KW fragments in three parts)
+// and multiplies them with its KW weight fragments of one column tile after the other; the 8 waves' partial tiles
 // are summed in wave order through one of two LDS buffers (one barrier per column tile: a buffer is written
 // again two tiles later, after the barrier that follows its readers), and wave r stores row tile r.
-// Measured (L10 H768, 70656 columns): 10 rows 21.3 -> 19.5 us (5.7 TB/s of weights and results; a large copy reaches 5.1), 80
-// rows 64.6 -> 30.9 us (4.2 TB/s) against one workgroup per 64 columns that held the weights and staged
-// silu(c) of every row tile anew (1104 workgroups x 5 tiles), with less error against 64 bits (2.5e-6 -> 1e-7 at up
-// to 48 rows, whose third part fits; the same above).
+// Measured (L10 H768, 70656 columns): 10 rows 21.3 -> 19.1 us (5.8 TB/s of weights and results; a large copy reaches 5.1), 80
+// rows 59.4 -> 31.3 us (4.2 TB/s), 160 rows 104 -> 51 us, against one workgroup per 64 columns that held the weights and
+// staged silu(c) of every row tile anew, in two parts (error against 64 bits 2.5e-6; three parts: 9e-8). With the third part
+// only where the registers hold it 80 rows take 29.5 us, and a row's bits depend on how many rows there are.
 template <int KT, int NRT>
 __global__ __launch_bounds__(64 * MODP_WAVES, NRT == 1 ? 4 : 2) void modproj_kernel(mkx_modproj_args a) {
-  constexpr int KW = KT / MODP_WAVES, PF = modp_ahead<KT, NRT>(), NS = modp_parts<NRT>();
+  constexpr int KW = KT / MODP_WAVES, PF = modp_ahead<KT, NRT>(), NS = MODP_PARTS;
   static_assert(KT % MODP_WAVES == 0 && NRT <= MODP_WAVES, "K splits over the waves; one wave stores a row tile");
+  constexpr int NL = modp_lds_tiles<KT, NRT>(), N3 = NRT - NL;  // row tiles from N3 on: third part in LDS
   __shared__ f32x4 part[2][MODP_WAVES][NRT][64];
+  __shared__ bf16x8 xl[NL ? MODP_WAVES : 1][NL ? NL : 1][KW][64];  // (each wave reads what it wrote)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int K = a.K, r0 = blockIdx.y * (16 * NRT), nct = a.N / 16;
-  const int ct0 = (int)((int64_t)nct * blockIdx.x / gridDim.x), ct1 = (int)((int64_t)nct * (blockIdx.x + 1) / gridDim.x);
+  const int K = a.K, r0 = (int)(blockIdx.x / MODP_XCDS) * (16 * NRT), nct = a.N / 16;
+  const int nr = gridDim.y * MODP_XCDS, range = blockIdx.y * MODP_XCDS + blockIdx.x % MODP_XCDS;
+  const int ct0 = (int)((int64_t)nct * range / nr), ct1 = (int)((int64_t)nct * (range + 1) / nr);
   // weight fragments of column tile ct: row 16 ct + (lane & 15), k = 32 t + 8 (lane >> 4) (fragment order: one
   // contiguous KW KB block per wave and tile; row-major: 16 rows x 64 KW B)
   const bool fo = a.w_fragment_order != 0;
@@ -102,15 +114,20 @@ __global__ __launch_bounds__(64 * MODP_WAVES, NRT == 1 ? 4 : 2) void modproj_ker
 #pragma unroll
     for (int s = 0; s < PF; ++s) load(s, ct0 + s);
   }
-  bf16x8 x[NRT][KW][NS];
+  bf16x8 x[NRT][KW][2], x3[N3][KW];
 #pragma unroll
   for (int r = 0; r < NRT; ++r) {
     const int row = min(r0 + 16 * r + (lane & 15), a.R - 1);  // rows past R repeat a valid row, never stored
     const float* cp = a.c + (int64_t)row * a.c_stride + 32 * KW * wave + 8 * (lane >> 4);
 #pragma unroll
-    for (int t = 0; t < KW; ++t)
-      modp_silu_split<NS>(*reinterpret_cast<const f32x4*>(cp + 32 * t), *reinterpret_cast<const f32x4*>(cp + 32 * t + 4),
-                          x[r][t]);
+    for (int t = 0; t < KW; ++t) {
+      bf16x8 f[NS];
+      modp_silu_split<NS>(*reinterpret_cast<const f32x4*>(cp + 32 * t), *reinterpret_cast<const f32x4*>(cp + 32 * t + 4), f);
+      x[r][t][0] = f[0];
+      x[r][t][1] = f[1];
+      if (r < N3) x3[r < N3 ? r : 0][t] = f[2];
+      else xl[wave][r - N3][t][lane] = f[2];
+    }
   }
   const int row = r0 + 16 * wave + (lane & 15);  // the row this lane stores (waves below NRT)
   const bool stores = wave < NRT && row < a.R;
@@ -124,7 +141,9 @@ __global__ __launch_bounds__(64 * MODP_WAVES, NRT == 1 ? 4 : 2) void modproj_ker
 #pragma unroll
       for (int t = 0; t < KW; ++t)
 #pragma unroll
-        for (int r = 0; r < NRT; ++r) acc[r] = mfma16(__builtin_bit_cast(bf16x8, wf[s][t]), x[r][t][i], acc[r]);
+        for (int r = 0; r < NRT; ++r)
+          acc[r] = mfma16(__builtin_bit_cast(bf16x8, wf[s][t]),
+                          i < 2 ? x[r][t][i & 1] : r < N3 ? x3[r < N3 ? r : 0][t] : xl[wave][r - N3][t][lane], acc[r]);
     load(s, ct + PF);
     const int buf = (ct - ct0) & 1;
 #pragma unroll

@@ -175,8 +175,8 @@ def _rand(*shape, seed, std=1.0):
                                      (129, 768, 16 * 259), (161, 1024, 16)])
 def test_modulations_row_and_column_edges(R, K, N, fragment_order):
     """Row tiles of every count a workgroup holds and more than one row group; fewer column tiles than workgroups,
-    and ranges that leave remainders of the weights' pipeline. Against 64 bits: silu(c) is held in two or
-    three bf16 parts (2^-18 relative at worst), a result is a sum of at most 3 K / 8 + 16 fp32 additions per wave and
+    and ranges that leave remainders of the weights' pipeline. Against 64 bits: silu(c) is held in three
+    bf16 parts (well within the 2^-18 of two), a result is a sum of at most 3 K / 8 + 16 fp32 additions per wave and
     over the waves, each rounded to 2^-24 of at most S = sum |silu(c) w| + |b|; the hardware exp and reciprocal add 2^-20."""
     c, w, b = _rand(R, K + 12, seed=R)[:, :K], _rand(N, K, seed=K, std=0.02).bfloat16(), _rand(N, seed=N, std=0.02)
     proj = ModulationProjection(w.cuda(), b.cuda(), fragment_order=fragment_order)
@@ -186,6 +186,17 @@ def test_modulations_row_and_column_edges(R, K, N, fragment_order):
     S = a.abs() @ w.double().abs().T + b.double().abs()
     bound = (2.0 ** -18 + 2.0 ** -20 + (3 * K / 8 + 16) * 2.0 ** -24) * S
     assert bool(((out - ref).abs() <= bound).all()), float(((out - ref).abs() / S).max())
+
+
+@pytest.mark.parametrize("K", [256, 512, 768, 1024])
+def test_modulations_rows_do_not_depend_on_their_number(K):
+    """A row's result is the same bits alone and among any number of rows (row tiles per workgroup and row groups differ)."""
+    w, b = _rand(16 * 259, K, seed=K, std=0.02).bfloat16(), _rand(16 * 259, seed=9, std=0.02)
+    c = _rand(161, K, seed=10).cuda()
+    proj = ModulationProjection(w.cuda(), b.cuda())
+    whole = proj(c)
+    for R in (1, 10, 17, 48, 49, 64, 65, 80, 81, 96, 97, 113, 128, 160):
+        assert torch.equal(proj(c[:R]), whole[:R]), R
 
 
 def _input_single_launch(step, N, sc):

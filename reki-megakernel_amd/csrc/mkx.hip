@@ -678,6 +678,9 @@ int mkx_run(mkx_handle* h, const mkx_step_args* a, void* stream_) {
         ((RTn + lay.rgs_cao - 1) / lay.rgs_cao) * NH > 256 || sk.HT > 64 || 6 * lay.rgs_qkv > 64 || lay.nred > 256)
       return fail(MKX_EUNSUPPORTED, "row grouping needs more than 256 ready epochs per wait");
     if (lay.lds_mods + a->B * 2 * H * 4 > sk.SMALL) return fail(MKX_EUNSUPPORTED, "GEMM LDS map does not fit");
+    // the row-wise kernels take these as constants
+    if (rows && (lay.nt_o != 1 || lay.nt_cao != 1 || lay.nt_down != 1 || lay.tpr != 1 || lay.nrg != lay.rgs_qkv))
+      return fail(MKX_EUNSUPPORTED, "the row-wise form takes tasks and reducers of one column tile, in the QKV stage's row groups");
   }
   if (h->profile && mkx_barriers(h, a->n_steps) + 1 > h->prof_len) return fail(MKX_EINVAL, "profile buffer shorter than barriers + 1");
 #ifdef MKX_TRACE

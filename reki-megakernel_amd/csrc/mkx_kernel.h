@@ -3431,7 +3431,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
     if (!d.first && S::RW && inproj) {
       const float* xn = c.xstep(d.s + 1);
       for (int it = c.tid; it < nrows * adim; it += NTHREADS) {
-        const int ri = (S::MDIV ? mdiv(it, p.m_adim) : it / adim), a = it - ri * adim;
+        const int ri = mdiv(it, p.m_adim), a = it - ri * adim;
         xp[it] = xn[(long long)ri * p.A + a];
       }
     } else if (!d.first) {
@@ -3552,7 +3552,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
 #pragma unroll
           for (int k = 0; k < IB; ++k) {
             const int row = min(row1 + k * (NTHREADS / 8), p.NRP - 1);
-            const int b = (S::MDIV ? mdiv(row, p.m_mqp) : row / p.Mqp), i = row - b * p.Mqp;
+            const int b = mdiv(row, p.m_mqp), i = row - b * p.Mqp;
             sc[k] = ldf4(c.modrow(min(b, p.B - 1), sn) + col);  // layer 0 self-attention AdaRMS scale
             const int ir = min(max(i - p.T, 0), max(p.R - 1, 0));  // (a valid register row, used for register rows only)
             rg[k] = p.R > 0 ? *reinterpret_cast<const uint2*>(p.reg_tok + (long long)ir * S::H + col) : uint2{0u, 0u};
@@ -3561,7 +3561,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
           for (int k = 0; k < IB; ++k) {
             const int row = row1 + k * (NTHREADS / 8);
             if (row >= p.NRP) break;
-            const int b = (S::MDIV ? mdiv(row, p.m_mqp) : row / p.Mqp), i = row - b * p.Mqp;
+            const int b = mdiv(row, p.m_mqp), i = row - b * p.Mqp;
             f32x4 v = {0.f, 0.f, 0.f, 0.f};
             if (b < p.B && i < p.T) {
               v = bv0;
@@ -3583,7 +3583,7 @@ __device__ __forceinline__ void tail_stage(Ctx<S>& c, const Desc& d, BarCtx& bc,
         // item: row, 4-column piece q of the task's tiles 2 t (q < 4) and 2 t + 1
         for (int it = c.tid; it < p.NRP * 8; it += NTHREADS) {
           const int row = it >> 3, q = it & 7;
-          const int b = (S::MDIV ? mdiv(row, p.m_mqp) : row / p.Mqp), i = row - b * p.Mqp;
+          const int b = row / p.Mqp, i = row - b * p.Mqp;
           const int col = t * 32 + 4 * q;
           f32x4 v, sc;
           uint2 rg;
@@ -3711,7 +3711,7 @@ __device__ __forceinline__ void prefetch(Ctx<S>& c, const Desc& d, const int* s_
 // into LDS, by waves 1-3
 template <class S>
 __device__ __forceinline__ void prefetch_shifts(Ctx<S>& c, const Desc& d) {
-  // (the row-wise form's tasks load their shift fragments after the poll)
+  // (the row-wise form's tasks load their shift fragments themselves, ahead of the poll)
   if (S::RW || c.wave == 0 || !(d.kind == K_QKV || d.kind == K_GU) || d.st == ST_TAIL || d.st == ST_SA || d.st == ST_CA ||
       task_first(c, d.pk) >= d.ntask)
     return;

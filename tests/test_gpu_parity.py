@@ -239,6 +239,26 @@ def test_tiny_single_row_tile_rowwise():
         _check_loop("tiny (row-wise GEMMs)", make_case(TINY))
 
 
+@pytest.mark.parametrize("form", ["rows", "passes"])
+@pytest.mark.parametrize("shape, dims", [({}, (24, 16, 17, 8, 1)), ({"H": 768, "NH": 12, "I": 3072, "T_act": 11}, (21, 17, 1))])
+def test_every_dim_of_x_for_every_group_of_action_dims(shape, dims, form):
+    """Action dims at, past and below the edge of the step tail's group of 16, over several steps, all 32 dims of x compared:
+    the real ones carry over from step to step, the padded ones hold the last step's dt v. One handle runs the wide cases
+    first, so the narrow ones find other values in the padded dims of the step areas (and of x itself)."""
+    with _gemm_form(form):
+        case = make_case(replace_cfg(TINY, B=3, **shape), random_mods=True)
+        mk = ExpertMegakernel(case["model"])
+        for adim in dims:
+            cfg = case["cfg"] = replace_cfg(case["cfg"], action_dim=adim)
+            x = mk.run(case["noise"], case["mods"], case["dt"], case["past"], adim)
+            mk.check()
+            ref = oracle_steps(case, case["noise"], 1, cfg.num_steps - 1, "fp32")
+            (m, a), (mall, aall) = diff(x, ref, adim), diff(x, ref, cfg.A)
+            _report("all dims", form=form, H=cfg.H, action_dim=adim, real_max=m, real_mean=a, all_max=mall, all_mean=aall)
+            assert float(ref[..., adim:].abs().max()) > 10 * TIGHT_MAX
+            assert mall <= TIGHT_MAX and aall <= TIGHT_MEAN, (adim, mall, aall)
+
+
 def test_barrier_count_invariant_and_determinism():
     case = make_case(TINY)
     cfg = case["cfg"]

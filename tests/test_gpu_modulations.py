@@ -236,3 +236,56 @@ def test_modulation_input_step_and_width_edges(N, B, H, tdim, workspace):
     bound = e_h1 @ t2w.to(d).abs().T + (3 * H / 4 + 16) * 2.0 ** -24 * (h1.abs() @ t2w.to(d).abs().T + t2b.to(d).abs())
     bound = bound[None] + 2.0 ** -22 * (1.0 + sc.to(d).abs()[:, None])
     assert bool(((out - ref).abs() <= bound).all()), float((out - ref).abs().max())
+
+
+@pytest.mark.parametrize("R, K, N", [(3, 256, 48), (20, 768, 16 * 300), (70, 512, 64), (70, 1024, 64), (100, 768, 32)])
+def test_modulations_padded_strides(R, K, N):
+    """Rows of c and of the result further apart than they are long: the same bits as with dense rows, nothing read from
+    the gaps (NaNs) and nothing written to them."""
+    w, b = _rand(N, K, seed=K, std=0.02).bfloat16().cuda(), _rand(N, seed=N, std=0.02).cuda()
+    dense = _rand(R, K, seed=R).cuda()
+    want = ModulationProjection(w, b, fragment_order=False)(dense)
+    cs, os_ = K + 20, N + 12
+    c, out = torch.full((R, cs), float("nan"), device="cuda"), torch.full((R + 1, os_), float("nan"), device="cuda")
+    c[:, :K] = dense
+    a = _lib.MkxModprojArgs(R=R, K=K, N=N, c=c.data_ptr(), c_stride=cs, w=w.data_ptr(), bias=b.data_ptr(), out=out.data_ptr(),
+                            out_stride=os_, w_fragment_order=0)
+    _lib.check(_lib.lib().mkx_modulations(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
+               "mkx_modulations")
+    torch.cuda.synchronize()
+    assert torch.equal(out[:R, :N], want)
+    assert bool(torch.isnan(out[:, N:]).all() and torch.isnan(out[R]).all())
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("N, B, H, tdim", [(1, 1, 256, 32), (10, 3, 768, 256), (17, 2, 512, 96), (16, 5, 1024, 512)])
+def test_modulation_input_padded_strides(N, B, H, tdim, workspace):
+    """state_cond rows, steps and samples further apart than dense: the same bits, gaps neither read nor written, and no
+    float past the workspace's N * H."""
+    bf = torch.bfloat16
+    t1w, t2w = _rand(H, tdim, seed=1, std=0.05).to(bf).cuda(), _rand(H, H, seed=2, std=0.05).to(bf).cuda()
+    t1b, t2b, sc = _rand(H, seed=3, std=0.1).cuda(), _rand(H, seed=4, std=0.1).cuda(), _rand(B, H, seed=5).cuda()
+    lib, stream = _lib.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def run(s, out, sc_stride, sb, sk):
+        a = _lib.MkxModinArgs(N=N, B=B, H=H, tdim=tdim, t1_w=t1w.data_ptr(), t1_b=t1b.data_ptr(), t2_w=t2w.data_ptr(),
+                              t2_b=t2b.data_ptr(), state_cond=s.data_ptr(), sc_stride=sc_stride, out=out.data_ptr(),
+                              out_stride_b=sb, out_stride_k=sk)
+        if workspace:
+            ws = torch.full((N * H + 64,), float("nan"), device="cuda")
+            _lib.check(lib.mkx_modulation_input_ws(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), stream), "mkx_modulation_input_ws")
+            torch.cuda.synchronize()
+            assert bool(torch.isfinite(ws[:N * H]).all() and torch.isnan(ws[N * H:]).all())
+        else:
+            _lib.check(lib.mkx_modulation_input(ctypes.byref(a), stream), "mkx_modulation_input")
+            torch.cuda.synchronize()
+        return out
+
+    want = run(sc, torch.empty(B, N, H, device="cuda"), H, N * H, H)
+    cs, sk, pad = H + 8, H + 20, 36
+    wide = torch.full((B, cs), float("nan"), device="cuda")
+    wide[:, :H] = sc
+    got = run(wide, torch.full((B + 1, N * sk + pad), float("nan"), device="cuda"), cs, N * sk + pad, sk)
+    rows = got[:B, :N * sk].view(B, N, sk)
+    assert torch.equal(rows[..., :H], want)
+    assert bool(torch.isnan(rows[..., H:]).all() and torch.isnan(got[:, N * sk:]).all() and torch.isnan(got[B]).all())

@@ -187,7 +187,6 @@ constexpr int MODIN_BLOCK = 1024;
 constexpr int MODIN_WAVES = MODIN_BLOCK / 64;
 constexpr int MODIN_KS = MODIN_WAVES / 4;  // waves sharing one 16-column tile of c, each over 1 / 4 of K
 constexpr int MODIN_MAX_TKB = 16;  // tdim <= 512
-constexpr int MODIN_MAX_HKB = 32;  // H <= 1024
 constexpr int MODIN_CK = 2;        // k-blocks of W1 loaded together
 constexpr int MODIN_NS = 3;        // bf16 parts of the embedding and of h1: as exact as fp32
 // dynamic LDS: the fragments of temb (later the K parts of c) and of h1

@@ -28,13 +28,12 @@ def rope_table(n: int, hd: int = 64, theta: float = 10000.0, device="cuda"):
     return torch.cos(emb).float().to(device), torch.sin(emb).float().to(device)
 
 
-def _caches(L: int, shape: tuple, device):
-    """(storage, [(K, V)] per layer): 2 L caches of `shape` in one allocation (2 L of them took longer on the host than the
-    launches run: 44 us a call against 25), layer l's K at l and V at L + l. unsafe_split: tensors of their own to autograd,
-    with in-place changes and version counters that the other caches know nothing of."""
-    kv = torch.empty(2 * L * shape[0], *shape[1:], dtype=torch.bfloat16, device=device)
-    parts = torch.unsafe_split(kv, shape[0])
-    return kv, list(zip(parts[:L], parts[L:]))
+def _layer_caches(kv: torch.Tensor, L: int) -> list:
+    """[(K, V)] per layer of the 2 L caches that lie one after the other in `kv`, layer l's K at l and V at L + l.
+    unsafe_split: tensors of their own to autograd, with in-place changes and version counters that the other caches know
+    nothing of."""
+    parts = torch.unsafe_split(kv, kv.shape[0] // (2 * L))
+    return list(zip(parts[:L], parts[L:]))
 
 
 class SourcePrepare:
@@ -106,7 +105,10 @@ class SourcePrepare:
         cal = torch.as_tensor(ca_len, dtype=torch.int32).reshape(-1).to(dev).contiguous()
         if cal.numel() != B:
             raise ValueError("ca_len needs one entry per sample")
-        kv, layers = _caches(self.L, (B, SP, self.NH, 64) if batched else (SP, self.NH, 64), dev)
+        # every layer's caches in one allocation (2 L of them took longer on the host than the launches run: 44 us a call
+        # against 25), taken apart once the launches are on their way
+        kv = torch.empty(2 * self.L * (B if batched else SP), *((SP,) if batched else ()), self.NH, 64, dtype=torch.bfloat16,
+                         device=dev)
         base, step = kv.data_ptr(), B * SP * self.NH * 64 * 2
         a = MkxSourceArgs(B=B, SP=SP)
         a.ctx, a.ca_len = x.data_ptr(), cal.data_ptr()
@@ -118,4 +120,4 @@ class SourcePrepare:
         check(fn(self._h, ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
               "mkx_source_run_noalloc" if static_scratch else "mkx_source_run")
         self._keep = (x, cal, cos, sin)  # inputs outlive the asynchronous launch
-        return layers
+        return _layer_caches(kv, self.L)

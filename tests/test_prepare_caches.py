@@ -3,14 +3,15 @@ place, also by something that requires a gradient, without a word to the others.
 import pytest
 import torch
 
-from mkx.prepare import _caches
+from mkx.prepare import _layer_caches
 
 
 @pytest.mark.parametrize("grad", [True, False])
 @pytest.mark.parametrize("shape", [(3, 5, 2, 64), (5, 2, 64)])
 def test_caches_are_tensors_of_their_own(shape, grad):
     with torch.set_grad_enabled(grad):
-        kv, layers = _caches(4, shape, "cpu")
+        kv = torch.empty(2 * 4 * shape[0], *shape[1:], dtype=torch.bfloat16)
+        layers = _layer_caches(kv, 4)
     flat = [t for pair in zip(*layers) for t in pair]  # K of every layer, then V
     assert len(layers) == 4 and len(flat) == 8
     for i, t in enumerate(flat):

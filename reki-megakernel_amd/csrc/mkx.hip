@@ -958,12 +958,15 @@ void modproj_launch(const mkx_modproj_args& a, hipStream_t stream) {
   const int nrt = (a.R + 15) / 16, MAX = nrt == 4 && KT <= 24 ? 2 : modp_max_nrt<KT>();
   const int ngr0 = (nrt + MAX - 1) / MAX, per = (nrt + ngr0 - 1) / ngr0, ngr = (nrt + per - 1) / per;
   const int slots = per == 1 ? 2 * MODP_GRID : MODP_GRID, nct = a.N / 16;
-  int y = 1;
-  long long best = -1;
-  for (int i = 1; i * MODP_XCDS <= slots; ++i) {
-    const int nr = i * MODP_XCDS;
-    const long long cost = ((long long)nr * ngr + slots - 1) / slots * ((nct + nr - 1) / nr + MODP_FIXED);
-    if (best < 0 || cost <= best) { best = cost; y = i; }
+  const int most = std::min(slots, nct + MODP_XCDS - 1) / MODP_XCDS;
+  int y = most;  // (one group: one round whatever the number)
+  if (ngr > 1) {
+    long long best = -1;
+    for (int i = 1; i <= most; ++i) {
+      const int nr = i * MODP_XCDS;
+      const long long cost = (long long)((nr * ngr + slots - 1) / slots) * ((nct + nr - 1) / nr + MODP_FIXED);
+      if (best < 0 || cost <= best) { best = cost; y = i; }
+    }
   }
   const dim3 grid((unsigned)(MODP_XCDS * ngr), (unsigned)y), block(64 * MODP_WAVES);
   switch (per) {

@@ -65,7 +65,7 @@ template <int KT, int NRT>
 constexpr int modp_ahead() { return NRT > 1 ? 2 : KT <= 8 ? 8 : KT <= 24 ? 4 : 3; }
 
 // row tiles of 16 that a workgroup holds at most, and the number of them whose third part lies in LDS: what the registers
-// do not hold of the 15 to 20 KB per row tile and wave (K 768, 80 rows: 32.3 us with none in LDS, 31.4 with one tile)
+// do not hold of the KW * 3 KB per row tile and wave (K 768, 80 rows: 32.3 us with none in LDS, 31.4 with one tile)
 template <int KT>
 constexpr int modp_max_nrt() { return KT <= 24 ? 5 : 4; }
 template <int KT, int NRT>

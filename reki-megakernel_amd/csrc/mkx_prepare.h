@@ -242,8 +242,8 @@ __device__ __forceinline__ void prep_unit(const PrepUnit& q, const SourceParams&
 // wave does not stand at a full load queue. Rows past a sample's valid length are zero in the result: the row
 // groups' workgroups share the stores of them. At most 5 row tiles, so that two workgroups share a CU (256 registers a
 // wave) and one's first loads and epilogue run beside the other's MFMAs.
-// Measured (10 layers, 12 heads, C 2048): one call of 300 rows 44.4 -> 30.5 us (619 TFLOP/s; a large matrix product
-// reaches 1115), eight of 300 down to 41 rows 183.6 -> 119.5 us, of which the numbering of the valid rows gives the
+// Measured (10 layers, 12 heads, C 2048): one call of 300 rows 44.4 -> 31 us (609 TFLOP/s; a large matrix product
+// reaches 1115), eight of 300 down to 41 rows 183.6 -> 120 us, of which the numbering of the valid rows gives the
 // larger part. No unit is full there: the matrix cores are busy 29 % of the time, operands come at 25 bytes per cycle and CU
 // (an L2-resident stream alone reaches 46 to 56), and the waves spend 39 % of theirs waiting for operands and 32 %
 // waiting to issue: 2160 workgroups in 4.2 rounds of two per CU, each with a start and an epilogue of its own.
